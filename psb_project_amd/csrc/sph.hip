@@ -18,6 +18,8 @@
 
 namespace psb {
 
+constexpr int kWide = 8;   // list entries per round of the density pass
+
 // Density from an existing list (standalone evaluate_densities_forces);
 // copies x, v into the scratch vec4 arrays with their w lanes filled.
 __global__ __launch_bounds__(256) void k_density_list(uint32_t n, Consts c,
@@ -34,13 +36,26 @@ __global__ __launch_bounds__(256) void k_density_list(uint32_t n, Consts c,
   const float4 xi = pos[p];
   float S = 0.f;
   const uint32_t m = cnt[p];
-  for (uint32_t k = 0; k < m; ++k) {
-    const float4 xj = pos[list[(uint64_t)k * n + p]];
+  auto add = [&](const float4& xj) {
     const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
     const float d2 = dot3(dx, dy, dz, dx, dy, dz);
     const float w = c.h2 - d2;
     S = __builtin_fmaf(w * w, w, S);
-  }
+  };
+  walk_list<kWide>(p, n, m, list, [&](const uint32_t (&q)[kWide]) {
+    float4 xq[kWide];
+#pragma unroll
+    for (int u = 0; u < kWide; ++u) xq[u] = gather4(pos, q[u]);
+#pragma unroll
+    for (int u = 0; u < kWide; ++u) add(xq[u]);
+  }, [&](const uint32_t (&q)[kWide], uint32_t r) {
+    float4 xq[kWide];
+#pragma unroll
+    for (int u = 0; u < kWide; ++u) xq[u] = gather4(pos, q[u]);
+#pragma unroll
+    for (int u = 0; u < kWide; ++u)
+      if ((uint32_t)u < r) add(xq[u]);
+  });
   const float r = S * c.mc;
   const float pr = eos(c, r);
   rho[p] = r;

@@ -1,0 +1,70 @@
+"""The list walkers at the edges of their rounds: particles with 0 to 40
+neighbours in one wave (a random cloud), list capacities around a round's
+length, and particle counts around a wave's; bitwise against the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from psb_project_amd import scenes
+from psb_project_amd._lib import MODE_CONFIG, MODE_REFERENCE, check, lib
+from tests.test_gpu_parity import gpu_grid_and_neighbors
+
+pytestmark = pytest.mark.gpu
+
+
+def cloud(n, seed, scale=1.0):
+    """Random positions, denser towards one corner: counts from 1 upwards."""
+    rng = np.random.default_rng(seed)
+    x = np.zeros((n, 4), np.float32)
+    side = scale * 0.02 * (n / 4.0) ** (1.0 / 3.0)
+    x[:, :3] = 0.01 + side * rng.random((n, 3)) ** 1.7
+    return x
+
+
+@pytest.mark.parametrize("mode", [MODE_REFERENCE, MODE_CONFIG])
+@pytest.mark.parametrize("n,cap", [(1, 4), (63, 1), (65, 7), (129, 8), (700, 9), (3000, 17), (3000, 64)])
+def test_densities_forces_on_uneven_lists(ctx, oracle, n, cap, mode):
+    p = scenes.wcsph_dam_break(n_side=20, mode=mode).params
+    x = cloud(n, 40 + n)
+    r = gpu_grid_and_neighbors(ctx, x, p.grid, p.support_radius, cap)
+    rng = np.random.default_rng(5)
+    vel = np.zeros((n, 4), np.float32)
+    vel[:, :3] = rng.normal(scale=0.2, size=(n, 3))
+    dvel = ctx.to_device(vel)
+    outs = {k: ctx.array(16 * n) for k in ("normals", "fP", "fV", "fS", "F")}
+    rho, prs = ctx.array(4 * n), ctx.array(4 * n)
+    check(lib().psb_evaluate_densities_forces(
+        ctx.handle, C.byref(p), r["nb"], r["bufs"][1].ptr, dvel.ptr, n, rho.ptr, prs.ptr,
+        outs["normals"].ptr, outs["fP"].ptr, outs["fV"].ptr, outs["fS"].ptr, outs["F"].ptr))
+    ref = oracle.evaluate_densities_forces(p, r["count"], r["list"].ravel(), r["xs"], vel)
+    assert np.array_equal(rho.download(np.float32, n), ref["density"])
+    assert np.array_equal(prs.download(np.float32, n), ref["pressure"])
+    for k in outs:
+        assert np.array_equal(outs[k].download(np.float32, (n, 4))[:, :3], ref[k][:, :3]), k
+
+
+@pytest.mark.parametrize("mode", [MODE_REFERENCE, MODE_CONFIG])
+@pytest.mark.parametrize("n", [1, 63, 129, 3000])
+@pytest.mark.parametrize("lanes", [1, 2])
+def test_pcisph_steps_on_uneven_lists(ctx, oracle, n, mode, lanes):
+    """One and two lanes per particle over the 32-bit list."""
+    from psb_project_amd.system import FluidSystem
+    p = scenes.pcisph_dam_break(n_side=1, s=0.01, mode=mode, retry_levels=0).params
+    p.max_neighbors = 33
+    p.max_iterations = 4
+    x = cloud(n, 90 + n)
+    g, o = FluidSystem(ctx, p, n), oracle.OracleSystem(p, n)
+    g.set_compact_list(False)
+    g.set_corrector_lanes(lanes)
+    g.set_particles(x)
+    o.set_particles(x)
+    for _ in range(2):
+        g.update(1)
+        o.update(1)
+        a, b = g.state(), o.state()
+        for k in ("pos", "vel", "vh", "density", "pressure", "ids"):
+            u, v = (a[k][:, :3], b[k][:, :3]) if a[k].ndim == 2 else (a[k], b[k])
+            assert np.array_equal(u, v, equal_nan=True), k
+    g.close()
+    o.close()
