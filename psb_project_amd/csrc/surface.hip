@@ -6,14 +6,15 @@
 // marching cubes (MarchingCube_Kernel.cu:14-158).  Here, on the device:
 //
 //   k_bounds     min / max of the particle positions (order-independent)
+//   k_sorted     particles in the order of a uniform grid of cell r
 //   k_iso        field at each node, f = sum_j (r^2 - d_j^2)^3 / r^6 over
-//                the particles within r = h / scale, read through a
-//                uniform grid of cell r (27 cells), in sorted order
+//                the particles within r = h / scale (27 cells), in sorted
+//                order; one wave per 4 x 4 x 4 nodes
 //   k_edges      crossed grid edges (one end <= iso, the other not), three
 //                per node (+x, +y, +z); exclusive scan -> vertex numbers
 //   k_vertices   one vertex per crossed edge, vertexInterpolate_MarchingCube
 //                (MarchingCube_Kernel.cu:145-155), and its normal: the
-//                direction of -grad f
+//                direction of -grad f; one wave per 4 x 4 x 4 nodes
 //   k_cubes      case index and triangle count per cube; exclusive scan
 //   k_emit       triangles as vertex-index triples, cube by cube (x fastest)
 //
@@ -56,15 +57,24 @@ __global__ __launch_bounds__(256) void k_bounds_init(uint32_t* out) {
   if (threadIdx.x < 6) out[threadIdx.x] = threadIdx.x < 3 ? 0xFFFFFFFFu : 0u;
 }
 
+// At most kBoundsBlocks workgroups, each with one atomic per bound: all
+// atomics fall on one cache line, and one set per wave (4,096 waves at 262,144
+// particles) took 281 us against 10.
+constexpr uint32_t kBoundsBlocks = 128;
 __global__ __launch_bounds__(256) void k_bounds(uint32_t n, const float4* __restrict__ pos,
                                                 const uint32_t* __restrict__ ids, uint32_t limit,
                                                 uint32_t* __restrict__ out) {
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ uint32_t red[4][6];
   uint32_t lo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, hi[3] = {0u, 0u, 0u};
-  if (p < n && kept(ids, limit, p)) {
+  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+    if (!kept(ids, limit, p)) continue;
     const float4 x = pos[p];
     const float c[3] = {x.x, x.y, x.z};
-    for (int a = 0; a < 3; ++a) lo[a] = hi[a] = order_key(c[a]);
+    for (int a = 0; a < 3; ++a) {
+      const uint32_t k = order_key(c[a]);
+      lo[a] = min(lo[a], k);
+      hi[a] = max(hi[a], k);
+    }
   }
   for (int a = 0; a < 3; ++a) {
 #pragma unroll
@@ -72,12 +82,19 @@ __global__ __launch_bounds__(256) void k_bounds(uint32_t n, const float4* __rest
       lo[a] = min(lo[a], (uint32_t)__shfl_xor((int)lo[a], o, 64));
       hi[a] = max(hi[a], (uint32_t)__shfl_xor((int)hi[a], o, 64));
     }
-  }
-  if ((threadIdx.x & 63u) == 0) {
-    for (int a = 0; a < 3; ++a) {
-      if (lo[a] != 0xFFFFFFFFu) atomicMin(out + a, lo[a]);
-      if (hi[a] != 0u) atomicMax(out + 3 + a, hi[a]);
+    if ((threadIdx.x & 63u) == 0) {
+      red[threadIdx.x >> 6][a] = lo[a];
+      red[threadIdx.x >> 6][3 + a] = hi[a];
     }
+  }
+  __syncthreads();
+  const uint32_t a = threadIdx.x;
+  if (a < 3) {
+    const uint32_t v = min(min(red[0][a], red[1][a]), min(red[2][a], red[3][a]));
+    if (v != 0xFFFFFFFFu) atomicMin(out + a, v);
+  } else if (a < 6) {
+    const uint32_t v = max(max(red[0][a], red[1][a]), max(red[2][a], red[3][a]));
+    if (v != 0u) atomicMax(out + a, v);
   }
 }
 
@@ -94,48 +111,146 @@ __device__ __forceinline__ void node_pos(const NodeGrid& G, int i, int j, int k,
   z = G.oz + (float)k * G.cell;
 }
 
-// particles of the 3 x 3 x 3 cells around (x, y, z), rows of x-consecutive
-// cells in ascending (z, y), each row in sorted order
-template <class F>
-__device__ __forceinline__ void for_near(const GridDev& g, const uint32_t* __restrict__ start,
-                                         const uint32_t* __restrict__ perm, float x, float y,
-                                         float z, F&& f) {
+// Positions in the grid's sorted order; a particle that is left out goes far
+// away (finite, so that its zero weight makes no NaN).
+constexpr float kFar = 1e18f;
+__global__ __launch_bounds__(256) void k_sorted(uint32_t n, const uint32_t* __restrict__ perm,
+                                                const float4* __restrict__ pos,
+                                                const uint32_t* __restrict__ ids, uint32_t limit,
+                                                float4* __restrict__ xs) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const uint32_t p = perm[k];
+  const float4 q = pos[p];
+  xs[k] = kept(ids, limit, p) ? make_float4(q.x, q.y, q.z, 0.f) : make_float4(kFar, kFar, kFar, 0.f);
+}
+
+// A wave's block of kNodeBlock^3 nodes and the box [lo, hi] around the points
+// its lanes evaluate.
+constexpr int kNodeBlock = 4;
+struct WaveBox {
+  float lo[3], hi[3];
+  int c0[3], c1[3];     // grid cells of the box's corners
+};
+
+__device__ __forceinline__ void box_cells(const GridDev& g, WaveBox& w) {
   uint32_t bad = 0;
-  const int cx = cell_coord(x, g.minx, g.cell, g.nx, bad);
-  const int cy = cell_coord(y, g.miny, g.cell, g.ny, bad);
-  const int cz = cell_coord(z, g.minz, g.cell, g.nz, bad);
-  const int x0 = max(cx - 1, 0), x1 = min(cx + 1, g.nx - 1);
-  for (int zz = max(cz - 1, 0); zz <= min(cz + 1, g.nz - 1); ++zz)
-    for (int yy = max(cy - 1, 0); yy <= min(cy + 1, g.ny - 1); ++yy) {
+  const float mn[3] = {g.minx, g.miny, g.minz};
+  const int nc[3] = {g.nx, g.ny, g.nz};
+  for (int a = 0; a < 3; ++a) {
+    w.c0[a] = max(cell_coord(w.lo[a], mn[a], g.cell, nc[a], bad) - 1, 0);
+    w.c1[a] = min(cell_coord(w.hi[a], mn[a], g.cell, nc[a], bad) + 1, nc[a] - 1);
+  }
+}
+
+// Visit, in sorted order, the particles near a wave's box: rows of cells in
+// ascending (z, y), 64 candidates at a time, one per lane; those within reach
+// of the box go to LDS in order, and every lane then sees each of them (an
+// LDS broadcast).  The field and normal sums of a lane's own 27 cells are
+// ~780 candidates at r = 3 spacings of which ~120 lie within r; per wave ~620
+// are near a block of 4^3 nodes, and one load serves 64 nodes instead of a
+// gather (through the permutation) per candidate and node.  262,144 particles,
+// 440,000 nodes: k_iso 617 -> 106 us, k_vertices 245 -> 57 us; what is left
+// is the ~13 VALU instructions per wave and survivor.
+template <class F>
+__device__ __forceinline__ void for_near_box(const GridDev& g, const uint32_t* __restrict__ start,
+                                             const float4* __restrict__ xs, const WaveBox& w,
+                                             float r2, float4* lds, F&& f) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const float reach2 = r2 * 1.001f;   // the box test is conservative, the sums decide
+  for (int zz = w.c0[2]; zz <= w.c1[2]; ++zz)
+    for (int yy = w.c0[1]; yy <= w.c1[1]; ++yy) {
       const uint64_t base = (uint64_t)g.nx * ((uint64_t)yy + (uint64_t)g.ny * (uint64_t)zz);
-      const uint32_t q1 = start[base + x1 + 1];
-      for (uint32_t q = start[base + x0]; q < q1; ++q) f(perm[q]);
+      const uint32_t q1 = start[base + w.c1[0] + 1];
+      for (uint32_t q0 = start[base + w.c0[0]]; q0 < q1; q0 += 64u) {
+        const uint32_t q = q0 + lane;
+        float4 x = make_float4(kFar, kFar, kFar, 0.f);
+        if (q < q1) x = xs[q];
+        const float dx = fmaxf(fmaxf(w.lo[0] - x.x, x.x - w.hi[0]), 0.f);
+        const float dy = fmaxf(fmaxf(w.lo[1] - x.y, x.y - w.hi[1]), 0.f);
+        const float dz = fmaxf(fmaxf(w.lo[2] - x.z, x.z - w.hi[2]), 0.f);
+        const bool in = dot3(dx, dy, dz, dx, dy, dz) <= reach2;
+        const uint64_t m = __ballot(in);
+        const uint32_t ns = (uint32_t)__popcll(m);
+        if (!ns) continue;
+        if (in) lds[__popcll(m & ((1ull << lane) - 1ull))] = x;
+        if (lane < 4u) lds[ns + lane] = make_float4(kFar, kFar, kFar, 0.f);   // pad to fours
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t k = 0; k < ns; k += 4u) {
+          float4 c[4];
+#pragma unroll
+          for (uint32_t u = 0; u < 4u; ++u) c[u] = lds[k + u];
+#pragma unroll
+          for (uint32_t u = 0; u < 4u; ++u) f(c[u]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     }
 }
 
-__global__ __launch_bounds__(256) void k_iso(NodeGrid G, GridDev g, const uint32_t* __restrict__ start,
-                                             const uint32_t* __restrict__ perm,
-                                             const float4* __restrict__ pos,
-                                             const uint32_t* __restrict__ ids, uint32_t limit,
-                                             float* __restrict__ iso) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t nn = (uint64_t)G.nx * G.ny * G.nz;
-  if (t >= nn) return;
-  const int i = (int)(t % G.nx), j = (int)((t / G.nx) % G.ny), k = (int)(t / ((uint64_t)G.nx * G.ny));
+// Whether particle x lies in the 27 cells around the point whose cell is c.  A
+// particle outside them is more than a cell (r) away but for rounding at the
+// cell borders: only a distance this close to r needs the test.
+constexpr float kNearEdge = 0.999f;
+__device__ __forceinline__ bool in_cells(const GridDev& g, const int (&c)[3], const float4& x) {
+  uint32_t bad = 0;
+  const int kx = cell_coord(x.x, g.minx, g.cell, g.nx, bad);
+  const int ky = cell_coord(x.y, g.miny, g.cell, g.ny, bad);
+  const int kz = cell_coord(x.z, g.minz, g.cell, g.nz, bad);
+  return abs(kx - c[0]) <= 1 && abs(ky - c[1]) <= 1 && abs(kz - c[2]) <= 1;
+}
+__device__ __forceinline__ void cells_of(const GridDev& g, float x, float y, float z, int (&c)[3]) {
+  uint32_t bad = 0;
+  c[0] = cell_coord(x, g.minx, g.cell, g.nx, bad);
+  c[1] = cell_coord(y, g.miny, g.cell, g.ny, bad);
+  c[2] = cell_coord(z, g.minz, g.cell, g.nz, bad);
+}
+
+// first node of wave `w`'s block (blocks x fastest), false past the last block
+__device__ __forceinline__ bool block_origin(const NodeGrid& G, uint32_t w, int (&o)[3]) {
+  const uint32_t bx = (G.nx + kNodeBlock - 1) / kNodeBlock, by = (G.ny + kNodeBlock - 1) / kNodeBlock,
+                 bz = (G.nz + kNodeBlock - 1) / kNodeBlock;
+  o[0] = (int)(w % bx) * kNodeBlock;
+  o[1] = (int)(w / bx % by) * kNodeBlock;
+  o[2] = (int)(w / (bx * by)) * kNodeBlock;
+  return w / (bx * by) < bz;
+}
+
+constexpr uint32_t kIsoWaves = 4;   // waves per workgroup, one node block each
+__global__ __launch_bounds__(64 * kIsoWaves) void k_iso(NodeGrid G, GridDev g,
+                                                        const uint32_t* __restrict__ start,
+                                                        const float4* __restrict__ xs,
+                                                        float* __restrict__ iso) {
+  __shared__ float4 lds[kIsoWaves][64 + 4];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int o[3];
+  if (!block_origin(G, blockIdx.x * kIsoWaves + wv, o)) return;
+  const int e[3] = {min(o[0] + kNodeBlock, G.nx) - 1, min(o[1] + kNodeBlock, G.ny) - 1,
+                    min(o[2] + kNodeBlock, G.nz) - 1};
+  WaveBox w;
+  node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
+  node_pos(G, e[0], e[1], e[2], w.hi[0], w.hi[1], w.hi[2]);
+  box_cells(g, w);
+  const int i = o[0] + (int)(lane & 3u), j = o[1] + (int)(lane >> 2 & 3u), k = o[2] + (int)(lane >> 4);
   float x, y, z;
   node_pos(G, i, j, k, x, y, z);
+  int c[3];
+  cells_of(g, x, y, z, c);
   float acc = 0.f;
-  for_near(g, start, perm, x, y, z, [&](uint32_t p) {
-    if (!kept(ids, limit, p)) return;
-    const float4 q = pos[p];
+  const float edge2 = G.r2 * kNearEdge;
+  for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
     const float dx = x - q.x, dy = y - q.y, dz = z - q.z;
     const float d2 = dot3(dx, dy, dz, dx, dy, dz);
-    if (d2 <= G.r2) {
-      const float w = G.r2 - d2;
-      acc = __builtin_fmaf(w * w, w, acc);
-    }
+    bool in = d2 <= G.r2;
+    if (__any(in && d2 > edge2)) in = in && (d2 <= edge2 || in_cells(g, c, q));
+    const float v = in ? G.r2 - d2 : 0.f;
+    acc = __builtin_fmaf(v * v, v, acc);   // v = 0 leaves acc (never -0) unchanged
   });
-  iso[t] = acc * G.inv_r6;
+  if (i < G.nx && j < G.ny && k < G.nz)
+    iso[(uint64_t)i + (uint64_t)G.nx * ((uint64_t)j + (uint64_t)G.ny * (uint64_t)k)] = acc * G.inv_r6;
 }
 
 __global__ __launch_bounds__(256) void k_edges(NodeGrid G, const float* __restrict__ iso,
@@ -154,32 +269,50 @@ __global__ __launch_bounds__(256) void k_edges(NodeGrid G, const float* __restri
   vcount[t] = __builtin_popcount(f);
 }
 
-__global__ __launch_bounds__(256) void k_vertices(NodeGrid G, GridDev g,
-                                                  const uint32_t* __restrict__ start,
-                                                  const uint32_t* __restrict__ perm,
-                                                  const float4* __restrict__ pos,
-                                                  const uint32_t* __restrict__ ids, uint32_t limit,
-                                                  const float* __restrict__ iso,
-                                                  const uint8_t* __restrict__ eflags,
-                                                  const uint32_t* __restrict__ vbase,
-                                                  float* __restrict__ verts,
-                                                  float* __restrict__ norms) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t nn = (uint64_t)G.nx * G.ny * G.nz;
-  if (t >= nn) return;
-  const uint32_t f = eflags[t];
-  if (!f) return;
-  const int i = (int)(t % G.nx), j = (int)((t / G.nx) % G.ny), k = (int)(t / ((uint64_t)G.nx * G.ny));
-  float ax, ay, az;
-  node_pos(G, i, j, k, ax, ay, az);
-  const float va = iso[t];
-  uint32_t v = vbase[t];
-  for (int axis = 0; axis < 3; ++axis) {
-    if (!(f >> axis & 1u)) continue;
-    const uint64_t tb = t + (axis == 0 ? 1 : axis == 1 ? (uint64_t)G.nx : (uint64_t)G.nx * G.ny);
-    float bx, by, bz;
-    node_pos(G, i + (axis == 0), j + (axis == 1), k + (axis == 2), bx, by, bz);
-    const float vb = iso[tb];
+// One wave per node block: the block's crossed edges are dealt to the lanes
+// (a wave of consecutive nodes had ~1 lane in 10 at work), 64 at a time.
+__global__ __launch_bounds__(64 * kIsoWaves) void k_vertices(
+    NodeGrid G, GridDev g, const uint32_t* __restrict__ start, const float4* __restrict__ xs,
+    const float* __restrict__ iso, const uint8_t* __restrict__ eflags,
+    const uint32_t* __restrict__ vbase, float* __restrict__ verts, float* __restrict__ norms) {
+  __shared__ float4 lds[kIsoWaves][64 + 4];
+  __shared__ uint8_t edge[kIsoWaves][192];   // node of the block (6 bits), axis (2 bits)
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int o[3];
+  if (!block_origin(G, blockIdx.x * kIsoWaves + wv, o)) return;
+  const int i = o[0] + (int)(lane & 3u), j = o[1] + (int)(lane >> 2 & 3u), k = o[2] + (int)(lane >> 4);
+  const uint64_t sy = (uint64_t)G.nx, sz = (uint64_t)G.nx * G.ny;
+  const uint64_t t0 = (uint64_t)o[0] + sy * (uint64_t)o[1] + sz * (uint64_t)o[2];
+  const uint32_t f = (i < G.nx && j < G.ny && k < G.nz)
+                         ? eflags[(uint64_t)i + sy * (uint64_t)j + sz * (uint64_t)k] : 0u;
+  uint32_t total = 0;
+#pragma unroll
+  for (uint32_t axis = 0; axis < 3u; ++axis) {
+    const uint64_t m = __ballot(f >> axis & 1u);
+    if (f >> axis & 1u)
+      edge[wv][total + __popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)(lane << 2 | axis);
+    total += (uint32_t)__popcll(m);
+  }
+  if (!total) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  WaveBox w;
+  node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
+  node_pos(G, o[0] + kNodeBlock, o[1] + kNodeBlock, o[2] + kNodeBlock, w.hi[0], w.hi[1], w.hi[2]);
+  box_cells(g, w);
+  const float edge2 = G.r2 * kNearEdge;
+  for (uint32_t v0 = 0; v0 < total; v0 += 64u) {
+    const bool on = v0 + lane < total;
+    const uint32_t ed = edge[wv][on ? v0 + lane : v0];
+    const int axis = (int)(ed & 3u);
+    const int ni = o[0] + (int)(ed >> 2 & 3u), nj = o[1] + (int)(ed >> 4 & 3u), nk = o[2] + (int)(ed >> 6);
+    const uint64_t t = t0 + (ed >> 2 & 3u) + sy * (ed >> 4 & 3u) + sz * (ed >> 6);
+    float ax, ay, az, bx, by, bz;
+    node_pos(G, ni, nj, nk, ax, ay, az);
+    node_pos(G, ni + (axis == 0), nj + (axis == 1), nk + (axis == 2), bx, by, bz);
+    const float va = iso[t], vb = iso[t + (axis == 0 ? 1 : axis == 1 ? sy : sz)];
+    const uint32_t v = vbase[t] + __builtin_popcount(eflags[t] & ((1u << axis) - 1u));
     float px, py, pz;
     // vertexInterpolate_MarchingCube (MarchingCube_Kernel.cu:145-155)
     if (fabsf(G.iso - va) < 0.000001f) { px = ax; py = ay; pz = az; }
@@ -190,25 +323,25 @@ __global__ __launch_bounds__(256) void k_vertices(NodeGrid G, GridDev g,
       px = ax + mu * (bx - ax); py = ay + mu * (by - ay); pz = az + mu * (bz - az);
     }
     // normal: -grad f ~ sum_j (x - x_j)(r^2 - d_j^2)^2, normalised
+    int c[3];
+    cells_of(g, px, py, pz, c);
     float gx = 0.f, gy = 0.f, gz = 0.f;
-    for_near(g, start, perm, px, py, pz, [&](uint32_t p) {
-      if (!kept(ids, limit, p)) return;
-      const float4 q = pos[p];
+    for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
       const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
       const float d2 = dot3(dx, dy, dz, dx, dy, dz);
-      if (d2 < G.r2) {
-        const float w = G.r2 - d2;
-        const float w2 = w * w;
-        gx = __builtin_fmaf(dx, w2, gx);
-        gy = __builtin_fmaf(dy, w2, gy);
-        gz = __builtin_fmaf(dz, w2, gz);
-      }
+      bool in = d2 < G.r2;
+      if (__any(in && d2 > edge2)) in = in && (d2 <= edge2 || in_cells(g, c, q));
+      const float u = in ? G.r2 - d2 : 0.f;
+      const float u2 = u * u;   // 0: adds a zero of either sign to sums that are never -0
+      gx = __builtin_fmaf(dx, u2, gx);
+      gy = __builtin_fmaf(dy, u2, gy);
+      gz = __builtin_fmaf(dz, u2, gz);
     });
+    if (!on) continue;
     const float gl = sqrtf(dot3(gx, gy, gz, gx, gy, gz));
     if (gl > 0.f) { gx = gx / gl; gy = gy / gl; gz = gz / gl; }
     verts[3 * (size_t)v] = px; verts[3 * (size_t)v + 1] = py; verts[3 * (size_t)v + 2] = pz;
     norms[3 * (size_t)v] = gx; norms[3 * (size_t)v + 1] = gy; norms[3 * (size_t)v + 2] = gz;
-    ++v;
   }
 }
 
@@ -279,7 +412,8 @@ struct psb_surface_s {
   uint64_t nodes = 0, cubes = 0;
   // element capacities of the device arrays below
   size_t cap_iso = 0, cap_ef = 0, cap_vc = 0, cap_vb = 0, cap_tc = 0, cap_tb = 0, cap_bs = 0;
-  size_t cap_v = 0, cap_n = 0, cap_t = 0;
+  size_t cap_v = 0, cap_n = 0, cap_t = 0, cap_xs = 0;
+  float4* xs = nullptr;            // positions in the grid's sorted order
   float* iso = nullptr;
   uint8_t* eflags = nullptr;
   uint32_t *vcount = nullptr, *vbase = nullptr, *tcount = nullptr, *tbase = nullptr;
@@ -364,7 +498,7 @@ psb_status psb_surface_destroy(psb_surface s) {
   if (s->grid) psb_finalize_grid(s->grid);
   for (void* p : {(void*)s->iso, (void*)s->eflags, (void*)s->vcount, (void*)s->vbase,
                   (void*)s->tcount, (void*)s->tbase, (void*)s->bsum, (void*)s->bounds,
-                  (void*)s->verts, (void*)s->norms, (void*)s->tris})
+                  (void*)s->verts, (void*)s->norms, (void*)s->tris, (void*)s->xs})
     if (p) (void)hipFree(p);
   if (s->h_counts) (void)hipHostFree(s->h_counts);
   delete s;
@@ -391,8 +525,8 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   if (!n) return PSB_OK;
   // bounds of the kept particles
   hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, st, s->bounds);
-  hipLaunchKernelGGL(k_bounds, dim3(blocks_for(n)), dim3(kBlock), 0, st, n, P, ids, id_limit,
-                     s->bounds);
+  hipLaunchKernelGGL(k_bounds, dim3(std::min(blocks_for(n), kBoundsBlocks)), dim3(kBlock), 0, st, n,
+                     P, ids, id_limit, s->bounds);
   PSB_HIP(hipGetLastError());
   PSB_HIP(hipMemcpyAsync(s->h_counts, s->bounds, 24, hipMemcpyDeviceToHost, st));
   PSB_HIP(hipStreamSynchronize(st));
@@ -451,9 +585,15 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   PSB_TRY(grow(s->tbase, s->cap_tb, s->cubes + 1));
   const uint64_t scan_tiles = (std::max(s->nodes, s->cubes) + kScanTile - 1) / kScanTile;
   PSB_TRY(grow(s->bsum, s->cap_bs, scan_tiles + 1));
+  PSB_TRY(grow(s->xs, s->cap_xs, n));
   const uint32_t nbn = blocks_for(s->nodes), nbc = blocks_for(s->cubes);
-  hipLaunchKernelGGL(k_iso, dim3(nbn), dim3(kBlock), 0, st, G, g, s->grid->start, s->grid->perm, P,
-                     ids, id_limit, s->iso);
+  uint32_t nbb = 1;   // node blocks, kIsoWaves to a workgroup
+  for (int a = 0; a < 3; ++a) nbb *= (dims[a] + kNodeBlock - 1) / kNodeBlock;
+  nbb = blocks_for(nbb, kIsoWaves);
+  hipLaunchKernelGGL(k_sorted, dim3(blocks_for(n)), dim3(kBlock), 0, st, n, s->grid->perm, P, ids,
+                     id_limit, s->xs);
+  hipLaunchKernelGGL(k_iso, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g, s->grid->start, s->xs,
+                     s->iso);
   hipLaunchKernelGGL(k_edges, dim3(nbn), dim3(kBlock), 0, st, G, s->iso, s->eflags, s->vcount);
   PSB_HIP(hipGetLastError());
   PSB_TRY(scan_exclusive(s->vcount, s->nodes, s->bsum, s->vbase, st));
@@ -470,9 +610,8 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   PSB_TRY(grow(s->verts, s->cap_v, 3 * (size_t)s->nv));
   PSB_TRY(grow(s->norms, s->cap_n, 3 * (size_t)s->nv));
   PSB_TRY(grow(s->tris, s->cap_t, 3 * (size_t)s->nt));
-  hipLaunchKernelGGL(k_vertices, dim3(nbn), dim3(kBlock), 0, st, G, g, s->grid->start,
-                     s->grid->perm, P, ids, id_limit, s->iso, s->eflags, s->vbase, s->verts,
-                     s->norms);
+  hipLaunchKernelGGL(k_vertices, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g, s->grid->start,
+                     s->xs, s->iso, s->eflags, s->vbase, s->verts, s->norms);
   if (s->cubes)
     hipLaunchKernelGGL(k_emit, dim3(nbc), dim3(kBlock), 0, st, G, s->iso, s->eflags, s->vbase,
                        s->tbase, s->tris);
