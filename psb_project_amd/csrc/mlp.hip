@@ -29,19 +29,20 @@ namespace psb {
 typedef bf16x4_t bf16x4;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint16_t f2bf(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-  u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
-  return (uint16_t)(u >> 16);
+// FP32 -> BF16, round to nearest even, on v_cvt_pk_bf16_f32 (an integer
+// sequence with its NaN branch was a third of the training pass's
+// instructions).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t f2bf2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
+__device__ __forceinline__ uint16_t f2bf(float x) { return (uint16_t)f2bf2(x, 0.f); }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
-  bf16x4 v;
-  v[0] = (short)f2bf(a); v[1] = (short)f2bf(b); v[2] = (short)f2bf(c); v[3] = (short)f2bf(d);
-  return v;
+  return __builtin_bit_cast(bf16x4, make_uint2(f2bf2(a, b), f2bf2(c, d)));
 }
 
 __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
@@ -81,23 +82,20 @@ __global__ void k_mlp_pack(const float* __restrict__ w, MlpFrags f) {
   if (t < kHid) f.w3[t] = bf2f(f2bf(w[kOffW3 + t]));
 }
 
-// Forward of one 16-sample tile.  xin(r, k) gives normalised input k of
-// sample r of the tile (0 for padding).  Outputs in D layout: z1/h1, z2/h2
+// Forward of one 16-sample tile.  a[j]: normalised input 4g + j of sample r
+// of the tile (0 for padding).  Outputs in D layout: z1/h1, z2/h2
 // [nt][j] = unit nt*16 + r of sample 4g + j; returns y for samples 4g + j in
 // lanes with r == 0 (other lanes hold partial sums).
 struct TileAct {
   f32x4 z1[4], z2[4], h1[4], h2[4];
+  f32x4 s1[4], s2[4];   // sigmoid(z), read again by the backward pass
   float y[4];
 };
 
-template <class XIN>
 __device__ __forceinline__ void tile_forward(const MlpFrags& f, const float* __restrict__ w,
-                                             XIN xin, uint16_t* lds, TileAct& t) {
+                                             const float (&a)[4], uint16_t* lds, TileAct& t) {
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
-  // layer 1: A1[r][4g+j] = x[r][4g+j]
-  float a[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) a[j] = xin(r, 4 * g + j);
+  // layer 1: A1[r][4g+j] = a[j] = x[r][4g+j]
   const bf16x4 A1 = pack4(a[0], a[1], a[2], a[3]);
   const float* b1 = w + kOffB1;
   const float* b2 = w + kOffB2;
@@ -109,7 +107,8 @@ __device__ __forceinline__ void tile_forward(const MlpFrags& f, const float* __r
     for (int j = 0; j < 4; ++j) {
       const float zz = z[j] + bias;
       t.z1[nt][j] = zz;
-      t.h1[nt][j] = zz * sigm(zz);
+      t.s1[nt][j] = sigm(zz);
+      t.h1[nt][j] = zz * t.s1[nt][j];
       lds[(4 * g + j) * kLdsRow + nt * 16 + r] = f2bf(t.h1[nt][j]);
     }
   }
@@ -132,7 +131,8 @@ __device__ __forceinline__ void tile_forward(const MlpFrags& f, const float* __r
     for (int j = 0; j < 4; ++j) {
       const float zz = z[j] + bias;
       t.z2[nt][j] = zz;
-      t.h2[nt][j] = zz * sigm(zz);
+      t.s2[nt][j] = sigm(zz);
+      t.h2[nt][j] = zz * t.s2[nt][j];
     }
   }
   // layer 3 (FP32 VALU): y[s] = sum_k h2[s][k] W3[k] + b3
@@ -162,14 +162,18 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float* __restrict__ fea
   const uint64_t tile = (uint64_t)blockIdx.x * 4 + wave;
   const uint64_t p0 = tile * 16;
   if (p0 >= n) return;   // whole wave exits together
-  auto xin = [&](int r, int k) -> float {
-    const uint64_t p = p0 + r;
-    if (k >= kIn || p >= n) return 0.f;
-    return (feat[(uint64_t)k * n + p] - nm.mu[k]) * nm.inv_sd[k];
-  };
-  TileAct t;
-  tile_forward(f, w, xin, lds, t);
   const int l = threadIdx.x & 63, g = l >> 4, r = l & 15;
+  float a[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    // clamped, so that the four loads go out together
+    const int k = min(4 * g + j, kIn - 1);
+    const uint64_t p = p0 + r < n ? p0 + r : n - 1u;
+    const float v = (feat[(uint64_t)k * n + p] - nm.mu[k]) * nm.inv_sd[k];
+    a[j] = (4 * g + j < kIn && p0 + r < n) ? v : 0.f;
+  }
+  TileAct t;
+  tile_forward(f, w, a, lds, t);
   if (r == 0) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -185,14 +189,15 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float* __restrict__ fea
   }
 }
 
-// Per-wave partial gradients: row w of part holds wave w's 4801 gradient
-// entries and its loss sum at kOffLoss; k_mlp_reduce adds the rows in wave
-// order, so a training run gives the same network every time.
+// Partial gradients: row b of part holds workgroup b's 4801 gradient entries
+// (its four waves' sums added in wave order) and its loss sum at kOffLoss;
+// k_mlp_update adds the rows in a fixed order, so a training run gives the
+// same network every time.
 constexpr int kOffLoss = kNumParams;
 constexpr int kPartRow = kNumParams + 1;
 
-// Forward + backward over a minibatch; each wave stores its gradient sums
-// (and loss sum) into its row of part.  Samples idx[b0 .. b0 + nb) of the
+// Forward + backward over a minibatch; each workgroup stores its gradient
+// sums (and loss sum) into its row of part.  Samples idx[b0 .. b0 + nb) of the
 // dataset (feature SoA [8][ns] + target[ns]); MSE on normalised targets.
 __global__ __launch_bounds__(256) void k_mlp_train(const float* __restrict__ feat,
                                                    const float* __restrict__ target, uint64_t ns,
@@ -217,25 +222,31 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float* __restrict__ fea
   const float inv_b = 1.0f / (float)nb;
   for (uint32_t tile = wave_id; tile < ntiles; tile += nwaves) {
     const uint32_t s0 = tile * 16;
-    auto sample = [&](int rr) -> int64_t {
-      const uint32_t b = s0 + rr;
-      return b < nb ? (int64_t)idx[b] : -1;
-    };
-    auto xin = [&](int rr, int k) -> float {
-      const int64_t s = sample(rr);
-      if (k >= kIn || s < 0) return 0.f;
-      return (feat[(uint64_t)k * ns + s] - nm.mu[k]) * nm.inv_sd[k];
-    };
+    // every load that depends on the sample indices goes out before the
+    // forward pass (padding reads the last sample and is masked)
+    const uint32_t sr = idx[min(s0 + r, nb - 1u)];
+    uint32_t sj[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sj[j] = idx[min(s0 + 4 * g + j, nb - 1u)];
+    float xa[4], xb[4], tg[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int k = min(4 * g + j, kIn - 1), kr = min(r, kIn - 1);
+      const float v = (feat[(uint64_t)k * ns + sr] - nm.mu[k]) * nm.inv_sd[k];
+      xa[j] = (4 * g + j < kIn && s0 + r < nb) ? v : 0.f;
+      const float u = (feat[(uint64_t)kr * ns + sj[j]] - nm.mu[kr]) * nm.inv_sd[kr];
+      xb[j] = (r < kIn && s0 + 4 * g + j < nb) ? u : 0.f;
+      tg[j] = target[sj[j]];
+    }
     TileAct t;
-    tile_forward(f, w, xin, lds, t);
+    tile_forward(f, w, xa, lds, t);
     // dy for the 4 samples 4g + j, broadcast from lane 16g
     float dy[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int64_t s = sample(4 * g + j);
       float d = 0.f;
-      if (s >= 0) {
-        const float e = t.y[j] - target[s];
+      if (s0 + 4 * g + j < nb) {
+        const float e = t.y[j] - tg[j];
         d = 2.0f * e * inv_b;
         if (r == 0) lsum += e * e;
       }
@@ -254,7 +265,7 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float* __restrict__ fea
       const float w3 = f.w3[nt * 16 + r];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float sg = sigm(t.z2[nt][j]);
+        const float sg = t.s2[nt][j];
         const float dsilu = sg * (1.0f + t.z2[nt][j] * (1.0f - sg));
         dz2[nt][j] = dy[j] * w3 * dsilu;
         gb2[nt] += dz2[nt][j];
@@ -292,89 +303,126 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float* __restrict__ fea
       for (int kt = 0; kt < 4; ++kt) dh = mfma(A2[kt], f.w2b[(kt * 4 + nt) * 64 + l], dh);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float sg = sigm(t.z1[nt][j]);
+        const float sg = t.s1[nt][j];
         const float dsilu = sg * (1.0f + t.z1[nt][j] * (1.0f - sg));
         dz1[nt][j] = dh[j] * dsilu;
         gb1[nt] += dz1[nt][j];
       }
     }
     // dW1[out][in] += sum_s dZ1[s][out] X[s][in]:  A = dZ1^T (D tile), B[s][in] = x
-    float xb[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) xb[j] = xin(4 * g + j, r);
     const bf16x4 Bx = pack4(xb[0], xb[1], xb[2], xb[3]);
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
       gW1[mt] = mfma(pack4(dz1[mt][0], dz1[mt][1], dz1[mt][2], dz1[mt][3]), Bx, gW1[mt]);
   }
-  // ---- flush: reduce over the 4 lane groups where needed; every entry of
-  // the wave's row is written by exactly one lane ----
-  float* row = part + (size_t)wave_id * kPartRow;
-  float* gw1p = row + kOffW1;
-  float* gw2p = row + kOffW2;
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int out = mt * 16 + 4 * g + j;
-      if (r < kIn) gw1p[out * kIn + r] = gW1[mt][j];
-#pragma unroll
-      for (int nk = 0; nk < 4; ++nk) gw2p[out * kHid + nk * 16 + r] = gW2[mt][nk][j];
-    }
-  }
+  // ---- flush: the waves add their sums into one LDS row, one after the
+  // other, and the workgroup writes it out in full lines.  A row per wave was
+  // 9.8 MB in 64-byte pieces for 512 waves, read back by the update: 23.8 us
+  // for this pass and 9.1 for that, against 27.6 and 4.1. ----
+  __shared__ float row[kPartRow];
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
-    float a = gb1[nt], b = gb2[nt], c = gw3[nt];
-    a += __shfl_xor(a, 16, 64); a += __shfl_xor(a, 32, 64);
-    b += __shfl_xor(b, 16, 64); b += __shfl_xor(b, 32, 64);
-    c += __shfl_xor(c, 16, 64); c += __shfl_xor(c, 32, 64);
-    if (g == 0) {
-      row[kOffB1 + nt * 16 + r] = a;
-      row[kOffB2 + nt * 16 + r] = b;
-      row[kOffW3 + nt * 16 + r] = c;
-    }
+    gb1[nt] += __shfl_xor(gb1[nt], 16, 64); gb1[nt] += __shfl_xor(gb1[nt], 32, 64);
+    gb2[nt] += __shfl_xor(gb2[nt], 16, 64); gb2[nt] += __shfl_xor(gb2[nt], 32, 64);
+    gw3[nt] += __shfl_xor(gw3[nt], 16, 64); gw3[nt] += __shfl_xor(gw3[nt], 32, 64);
   }
   gb3 += __shfl_xor(gb3, 16, 64); gb3 += __shfl_xor(gb3, 32, 64);
   lsum += __shfl_xor(lsum, 16, 64); lsum += __shfl_xor(lsum, 32, 64);
-  if (l == 0) {
-    row[kOffB3] = gb3;
-    row[kOffLoss] = lsum;
-  }
-}
-
-// grad[k] += sum over the waves' rows of part[w][k]; loss = the loss sum.
-// Fixed order: row w goes to accumulator w % 8 (eight loads in flight), the
-// accumulators are added pairwise.
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ part, uint32_t rows,
-                                                    float* __restrict__ grad,
-                                                    float* __restrict__ loss) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (uint32_t)kPartRow) return;
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  uint32_t w = 0;
-  for (; w + 8 <= rows; w += 8) {
+  for (uint32_t k = threadIdx.x; k < (uint32_t)kPartRow; k += blockDim.x) row[k] = 0.f;
+  for (int turn = 0; turn < 4; ++turn) {
+    __syncthreads();
+    if (wave != turn) continue;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc[u] += part[(size_t)(w + u) * kPartRow + k];
+    for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int out = mt * 16 + 4 * g + j;
+        if (r < kIn) row[kOffW1 + out * kIn + r] += gW1[mt][j];
+#pragma unroll
+        for (int nk = 0; nk < 4; ++nk) row[kOffW2 + out * kHid + nk * 16 + r] += gW2[mt][nk][j];
+      }
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) {
+        row[kOffB1 + nt * 16 + r] += gb1[nt];
+        row[kOffB2 + nt * 16 + r] += gb2[nt];
+        row[kOffW3 + nt * 16 + r] += gw3[nt];
+      }
+    }
+    if (l == 0) {
+      row[kOffB3] += gb3;
+      row[kOffLoss] += lsum;
+    }
   }
-  for (; w < rows; ++w) acc[w & 7u] += part[(size_t)w * kPartRow + k];
-  const float sum = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
-  if (k < (uint32_t)kNumParams) grad[k] = grad[k] + sum;
-  else *loss = sum;
+  __syncthreads();
+  float* dst = part + (size_t)blockIdx.x * kPartRow;
+  for (uint32_t k = threadIdx.x; k < (uint32_t)kPartRow; k += blockDim.x) dst[k] = row[k];
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master parameters; zeroes grad.
-__global__ void k_mlp_adam(float* __restrict__ w, float* __restrict__ grad, float* __restrict__ m1,
-                           float* __restrict__ m2, float lr, float b1, float b2, float eps,
-                           float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kNumParams) return;
-  const float gr = grad[i];
-  const float m = b1 * m1[i] + (1.0f - b1) * gr;
-  const float v = b2 * m2[i] + (1.0f - b2) * gr * gr;
-  m1[i] = m;
-  m2[i] = v;
-  w[i] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
-  grad[i] = 0.f;
+// The rest of a training step in one launch: grad[k] += sum over the
+// workgroups' rows of part[w][k], the loss sum, and with `apply` Adam (Kingma & Ba 2015) on
+// the FP32 master parameters, the gradient zeroed and the parameter's BF16
+// copies in the fragments rewritten.  Fixed order: row w goes to accumulator
+// w % 8, the accumulators are added pairwise; the eight accumulators of a
+// column are eight threads.  A batch of 8,192: 4.1 us, against 26 us for one
+// thread per column (19 workgroups walking 512 rows) and 10 us for Adam and
+// the fragments in launches of their own.
+constexpr uint32_t kUpdateCols = 32;   // columns per workgroup (128-byte rows)
+struct AdamArgs {
+  int apply;
+  float lr, b1, b2, eps, c1, c2;
+};
+__global__ __launch_bounds__(8 * kUpdateCols) void k_mlp_update(
+    const float* __restrict__ part, uint32_t rows, float* __restrict__ grad, float* loss,
+    float* __restrict__ w, float* __restrict__ m1, float* __restrict__ m2, MlpFrags f, AdamArgs a) {
+  __shared__ float acc8[8][kUpdateCols];
+  const uint32_t u = threadIdx.x / kUpdateCols, col = threadIdx.x % kUpdateCols;
+  const uint32_t k = blockIdx.x * kUpdateCols + col;
+  float acc = 0.f;
+  if (k < (uint32_t)kPartRow) {
+    const float* src = part + (size_t)u * kPartRow + k;
+    const size_t step = 8 * (size_t)kPartRow;
+    uint32_t r = u;
+    for (; r + 56u < rows; r += 64u, src += 8 * step) {   // 8 rows of this accumulator in flight
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = src[j * step];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc += v[j];
+    }
+    for (; r < rows; r += 8u, src += step) acc += *src;
+  }
+  acc8[u][col] = acc;
+  __syncthreads();
+  if (u != 0u || k >= (uint32_t)kPartRow) return;
+  const float sum = ((acc8[0][col] + acc8[1][col]) + (acc8[2][col] + acc8[3][col])) +
+                    ((acc8[4][col] + acc8[5][col]) + (acc8[6][col] + acc8[7][col]));
+  if (k == (uint32_t)kOffLoss) { *loss = sum; return; }
+  const float gr = grad[k] + sum;
+  if (!a.apply) { grad[k] = gr; return; }
+  const float m = a.b1 * m1[k] + (1.0f - a.b1) * gr;
+  const float v = a.b2 * m2[k] + (1.0f - a.b2) * gr * gr;
+  m1[k] = m;
+  m2[k] = v;
+  const float wn = w[k] - a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
+  w[k] = wn;
+  grad[k] = 0.f;
+  const uint16_t h = f2bf(wn);
+  if (k < (uint32_t)kOffB1) {
+    const uint32_t o = k / kIn, i = k % kIn;
+    reinterpret_cast<uint16_t*>(f.w1)[((o >> 4) * 64u + (i >> 2) * 16u + (o & 15u)) * 4u + (i & 3u)] = h;
+  } else if (k >= (uint32_t)kOffW2 && k < (uint32_t)kOffB2) {
+    const uint32_t o = (k - kOffW2) / kHid, i = (k - kOffW2) % kHid;
+    // element (o, i) as W2[row][4g + j] of tile (tr, tk): see k_mlp_pack
+    auto at = [](uint32_t row, uint32_t kk) {
+      return (((kk >> 4) * 4u + (row >> 4)) * 64u + (kk >> 2 & 3u) * 16u + (row & 15u)) * 4u + (kk & 3u);
+    };
+    reinterpret_cast<uint16_t*>(f.w2f)[at(o, i)] = h;
+    reinterpret_cast<uint16_t*>(f.w2b)[at(i, o)] = h;
+  } else if (k >= (uint32_t)kOffW3 && k < (uint32_t)kOffB3) {
+    f.w3[k - kOffW3] = bf2f(h);
+  }
 }
 
 }  // namespace psb
@@ -387,8 +435,9 @@ struct psb_mlp_s {
   float* grad = nullptr;   // [kNumParams]
   float* m1 = nullptr;
   float* m2 = nullptr;
-  float* loss = nullptr;   // [1]
-  float* part = nullptr;   // per-wave gradient rows of a training step
+  float* h_loss = nullptr; // host-mapped: the last training step's loss sum
+  float* d_loss = nullptr;
+  float* part = nullptr;   // per-workgroup gradient rows of a training step
   uint32_t part_rows = 0;
   MlpFrags frags{};
   void* frag_mem = nullptr;
@@ -433,7 +482,9 @@ psb_status psb_mlp_create(psb_context ctx, uint64_t seed, psb_mlp* out) {
   if ((e = hipMalloc(&m->grad, 4 * kNumParams)) != hipSuccess) return fail(e);
   if ((e = hipMalloc(&m->m1, 4 * kNumParams)) != hipSuccess) return fail(e);
   if ((e = hipMalloc(&m->m2, 4 * kNumParams)) != hipSuccess) return fail(e);
-  if ((e = hipMalloc(&m->loss, 64)) != hipSuccess) return fail(e);
+  if ((e = hipHostMalloc((void**)&m->h_loss, 64, hipHostMallocMapped | hipHostMallocCoherent)) != hipSuccess)
+    return fail(e);
+  if ((e = hipHostGetDevicePointer((void**)&m->d_loss, m->h_loss, 0)) != hipSuccess) return fail(e);
   const size_t fb = sizeof(bf16x4) * 64 * 36 + 4 * kHid;
   if ((e = hipMalloc(&m->frag_mem, fb)) != hipSuccess) return fail(e);
   bf16x4* fm = (bf16x4*)m->frag_mem;
@@ -467,7 +518,8 @@ psb_status psb_mlp_destroy(psb_mlp m) {
   if (!m) return PSB_OK;
   hipSetDevice(m->ctx->device);
   hipStreamSynchronize(m->ctx->stream);
-  hipFree(m->w); hipFree(m->grad); hipFree(m->m1); hipFree(m->m2); hipFree(m->loss);
+  hipFree(m->w); hipFree(m->grad); hipFree(m->m1); hipFree(m->m2);
+  if (m->h_loss) hipHostFree(m->h_loss);
   hipFree(m->frag_mem);
   if (m->part) hipFree(m->part);
   delete m;
@@ -522,7 +574,7 @@ psb_status psb_mlp_train_step(psb_mlp m, const float* features, const float* tar
   const uint32_t tiles = (batch + 15) / 16;
   uint32_t blocks = (tiles + 3) / 4;
   if (blocks > 512) blocks = 512;
-  const uint32_t rows = 4 * blocks;
+  const uint32_t rows = blocks;
   if (rows > m->part_rows) {
     PSB_HIP(hipStreamSynchronize(s));
     if (m->part) PSB_HIP(hipFree(m->part));
@@ -534,24 +586,24 @@ psb_status psb_mlp_train_step(psb_mlp m, const float* features, const float* tar
   hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(256), 0, s, features, targets, num_samples,
                      batch_idx, batch, m->w, m->frags, m->norm, m->part);
   PSB_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((kPartRow + 255) / 256), dim3(256), 0, s, m->part, rows,
-                     m->grad, m->loss);
-  PSB_HIP(hipGetLastError());
+  AdamArgs a{};
   if (apply_adam) {
     m->adam_t += 1;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = (float)(1.0 - std::pow(0.9, (double)m->adam_t));
-    const float c2 = (float)(1.0 - std::pow(0.999, (double)m->adam_t));
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kNumParams + 255) / 256), dim3(256), 0, s, m->w, m->grad,
-                       m->m1, m->m2, lr, b1, b2, 1e-8f, c1, c2);
-    PSB_HIP(hipGetLastError());
-    PSB_TRY(mlp_pack(m));
+    a.apply = 1;
+    a.lr = lr;
+    a.b1 = 0.9f;
+    a.b2 = 0.999f;
+    a.eps = 1e-8f;
+    a.c1 = (float)(1.0 - std::pow(0.9, (double)m->adam_t));
+    a.c2 = (float)(1.0 - std::pow(0.999, (double)m->adam_t));
   }
+  hipLaunchKernelGGL(k_mlp_update, dim3((kPartRow + kUpdateCols - 1) / kUpdateCols),
+                     dim3(8 * kUpdateCols), 0, s, m->part, rows, m->grad, m->d_loss, m->w, m->m1,
+                     m->m2, m->frags, a);
+  PSB_HIP(hipGetLastError());
   if (loss_out) {
-    float l = 0.f;
-    PSB_HIP(hipMemcpyAsync(&l, m->loss, 4, hipMemcpyDeviceToHost, s));
     PSB_HIP(hipStreamSynchronize(s));
-    *loss_out = l / (float)batch;
+    *loss_out = *(volatile float*)m->h_loss / (float)batch;
   }
   return PSB_OK;
 }

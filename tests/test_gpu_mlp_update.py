@@ -1,0 +1,51 @@
+"""The training step's update at the edges of its row groups: 1, 4, 8, 9, 64
+and 65 wave rows (batches of 16 samples a wave) and the most rows it takes,
+with and without Adam."""
+import numpy as np
+import pytest
+
+from psb_project_amd import learned
+from tests.test_gpu_learned import he_params
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch", [1, 17, 64, 144, 1024, 1030, 40000])
+def test_gradient_and_adam_of_one_step(ctx, oracle, batch):
+    rng = np.random.default_rng(batch)
+    ns = max(batch, 500)
+    feat = rng.normal(size=(8, ns)).astype(np.float32)
+    target = rng.normal(size=ns).astype(np.float32)
+    idx = rng.choice(ns, batch, replace=False).astype(np.uint32)
+    w = he_params(10)
+    df, dt, di = ctx.to_device(feat), ctx.to_device(target), ctx.to_device(idx)
+    mean, std = np.zeros(8, np.float32), np.ones(8, np.float32)
+    m = learned.PressureMLP(ctx)
+    m.set_params(w)
+    m.set_normalization(mean, std, 1.0)
+    loss = m.train_step(df.ptr, dt.ptr, ns, di.ptr, batch, apply_adam=False)
+    g = m.grad()
+    gref, lref = oracle.mlp_grad(w, mean, std, feat, target, idx, emulate_bf16=True)
+    assert loss == pytest.approx(lref, rel=1e-3)
+    assert np.linalg.norm(g - gref) / np.linalg.norm(gref) < 1e-2
+    # the same gradient through Adam: first step, bias-corrected moments
+    m.zero_grad()
+    m.train_step(df.ptr, dt.ptr, ns, di.ptr, batch, lr=1e-3)
+    f = np.float32
+    m1, m2 = (f(1) - f(0.9)) * g, (f(1) - f(0.999)) * g * g
+    want = w - f(1e-3) * (m1 / f(1 - 0.9)) / (np.sqrt(m2 / f(1 - 0.999)) + f(1e-8))
+    got = m.params()
+    assert np.allclose(got, want, rtol=0, atol=2e-7 * (1 + np.abs(w).max()))
+    assert not m.grad().any()
+    # the fragments hold the new weights: a fresh network given them agrees
+    out = [ctx.array(4 * ns) for _ in range(2)]
+    m.forward(df.ptr, ns, out[0].ptr)
+    k = learned.PressureMLP(ctx)
+    k.set_params(got)
+    k.set_normalization(mean, std, 1.0)
+    k.forward(df.ptr, ns, out[1].ptr)
+    ctx.sync()
+    a, b = (o.download(np.float32, ns) for o in out)
+    assert np.array_equal(a, b)
+    m.close()
+    k.close()
