@@ -802,12 +802,20 @@ static psb_status pci_sph_update_on(psb_context ctx, const psb_sph_params* prm, 
   b.aid = nullptr;
   const bool ref = prm->mode == PSB_MODE_REFERENCE;
   const bool warm = !ref && prm->warm_start == PSB_WARM_PREVIOUS;
-  PSB_TRY(launch_pci_reset(st, true, s));
   PSB_HIP(hipMemsetAsync(ctx->d_flags, 0, 4, s));
   // start density (PciSphSystem.cu:17), scratch copies with v.w = 1/rho
   PSB_TRY(launch_density_list(n, c, nb, reinterpret_cast<const float4*>(pos4),
                               reinterpret_cast<const float4*>(vel4), density, tmp_p, xs, vs, s));
   if (!warm) PSB_HIP(hipMemsetAsync(pressure, 0, 4 * (size_t)n, s));
+  // the start pressure is not read again: its n words hold the error slots
+  // (with one word for all workgroups' maxima the density pass took 23.4 us
+  // at 253,952 particles, now 18.2; 11.1 at 44,000, now 7.9)
+  ErrSlots es{};
+  if (n >= (uint32_t)(kErrSlots * kMaxIterSlots)) {
+    es.base = reinterpret_cast<uint32_t*>(tmp_p);
+    es.stride = n / kErrSlots;
+  }
+  PSB_TRY(launch_pci_reset(st, true, s, 1, nullptr, es));
   PciOut o{};
   o.normals = reinterpret_cast<float4*>(normals4);
   o.fV = reinterpret_cast<float4*>(f_viscosity4);
@@ -819,23 +827,31 @@ static psb_status pci_sph_update_on(psb_context ctx, const psb_sph_params* prm, 
   o.vav = reinterpret_cast<float4*>(vel_inter_av4);
   o.vap = reinterpret_cast<float4*>(vel_inter_ap4);
   o.flags = ctx->d_flags;
+  o.es = es;
   const bool surf = ref || prm->surface_tension != 0.f;
   PSB_TRY(launch_pci_nonpressure(n, c, surf, warm, true, nb.count, nb.list, xs, vs, density,
                                  b.avh, pressure, b, o, s));
   float4* cur = b.xp0;
   float4* nxt = xp1;
+  // Two lanes per particle while one leaves the chip short of waves (reference
+  // mode, density + force pass, one lane -> two: 729 particles 18.9 -> 13.9
+  // us, 32,768 21.7 -> 15.7, 85,184 24.2 -> 20.3, 140,608 28.6 -> 26.9;
+  // 195,112 30.6 -> 31.4, 253,952 35.1 -> 35.9)
+  int cus = 0;
+  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+  const int lanes = (uint64_t)n <= 640ull * (uint64_t)cus ? 2 : 1;
   if (warm) {
     PSB_TRY(launch_pci_force(n, c, false, nb.count, nb.list, cur, nxt, density, pressure, b, st, -1,
-                             1, o, s));
+                             1, o, s, lanes));
     std::swap(cur, nxt);
   }
   int iters = 0;
   float err = 0.f;
   for (int k = 0; k < c.max_it; ++k) {
     PSB_TRY(launch_pci_density(n, c, nb.count, nb.list, cur, pressure, density, b.dl, st, k,
-                               nullptr, 0, s));
+                               nullptr, 0, s, nullptr, lanes, nullptr, es));
     PSB_TRY(launch_pci_force(n, c, false, nb.count, nb.list, cur, nxt, density, pressure, b, st, k,
-                             0, o, s));
+                             0, o, s, lanes));
     std::swap(cur, nxt);
     if (k + 1 >= c.min_it) {
       PSB_HIP(hipMemcpyAsync(ctx->h_pinned, st, 16, hipMemcpyDeviceToHost, s));

@@ -937,18 +937,31 @@ __device__ __forceinline__ void for_neighbors_split(uint32_t p, uint32_t n, uint
         if ((uint32_t)u < r) f(u & 1, xq[u]);
     });
   } else {
+    // the plain list, lane l taking the entries k = l (mod 2), the next
+    // round's entries (clamped to the particle's own) loaded ahead
+    auto row = [&](uint32_t k) { return list.at(min(k, m - 1u), p); };
+    if (m <= lane) return;
+    uint32_t nx[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) nx[u] = row(lane + 2u * u);
     uint32_t k = lane;
     for (; k + 2 * (U - 1) < m; k += 2 * U) {
-      uint32_t q[U];
       float4 xq[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) q[u] = list.at(k + 2 * u, p);
+      for (int u = 0; u < U; ++u) xq[u] = gather4(X, nx[u]);
 #pragma unroll
-      for (int u = 0; u < U; ++u) xq[u] = X[q[u]];
+      for (int u = 0; u < U; ++u) nx[u] = row(k + 2u * (U + u));
 #pragma unroll
       for (int u = 0; u < U; ++u) f(0, xq[u]);
     }
-    for (; k < m; k += 2) f(0, X[list.at(k, p)]);
+    if (k < m) {
+      float4 xq[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) xq[u] = gather4(X, nx[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k + 2u * u < m) f(0, xq[u]);
+    }
   }
 }
 
