@@ -722,8 +722,7 @@ psb_status psb_search_neighbors(psb_grid g, const float* sorted_pos4, uint32_t n
   GridDev gd = grid_dev(g->desc, radius);
   PSB_TRY(launch_neighbors(g, reinterpret_cast<const float4*>(sorted_pos4), n, radius * radius,
                            gd.R, nb, nullptr, 0.f, ctx->d_flags, ctx->d_flags + 1, ctx->stream));
-  PSB_HIP(hipMemcpyAsync(ctx->h_pinned, ctx->d_flags, 8, hipMemcpyDeviceToHost, ctx->stream));
-  PSB_HIP(hipMemcpyAsync(ctx->h_pinned + 2, g->flags, 4, hipMemcpyDeviceToHost, ctx->stream));
+  PSB_TRY(launch_words_out(ctx->d_flags, 2, g->flags, 1, nullptr, 0, ctx->d_pinned, ctx->stream));
   PSB_HIP(hipStreamSynchronize(ctx->stream));
   if (flags_out) *flags_out = ctx->h_pinned[0] | ctx->h_pinned[2];
   return PSB_OK;

@@ -116,6 +116,11 @@ constexpr size_t pci_update_scratch_bytes(size_t n) {
 // device with that device current (psb_init)
 psb_status static_scratch_setup(int device);
 
+// Start of an update call of one solve, in one launch: statistics, step
+// status and error slots reset, flags[0..1] and *grid_flags (when not null)
+// cleared.
+psb_status launch_pci_begin(PciStatus* st, ErrSlots es, uint32_t* flags, uint32_t* grid_flags,
+                            hipStream_t s);
 // one status per scene (scenes = 1 for a single system); done: batch counter
 psb_status launch_pci_reset(PciStatus* st, bool stats, hipStream_t s, uint32_t scenes = 1,
                             uint32_t* done = nullptr, ErrSlots es = ErrSlots{});
@@ -169,9 +174,10 @@ psb_status launch_pci_force_batch(const BatchMap& map, const Shape& sh, uint32_t
                                   const uint16_t* list16 = nullptr);
 
 // sph.hip
+// zero: cleared for every particle (may be null)
 psb_status launch_density_list(uint32_t n, const Consts& c, psb_neighbors nb, const float4* pos,
                                const float4* vel, float* rho, float* pres, float4* xs, float4* vs,
-                               hipStream_t s);
+                               float* zero, hipStream_t s);
 // the epilogue's arguments, for the fused path of launch_neighbors
 EpiArgs make_epilogue(const Consts& c, int pcisph, int warm, int xw_prev, float* pres,
                       const float* pprev, float4* xs, float4* vs, const uint32_t* ids);

@@ -39,8 +39,7 @@ __global__ void k_pci_retry_reset(PciStatus* st0, ErrSlots es, const uint32_t* s
   pci_reset_scene(st0, scenes ? scenes[blockIdx.x] : blockIdx.x, nullptr, es, true);
 }
 
-__global__ void k_pci_stats_reset(PciStatus* st0) {
-  PciStatus* st = st0 + blockIdx.x;
+__device__ __forceinline__ void pci_reset_stats(PciStatus* st) {
   if (threadIdx.x == 0) {
     st->total_iters = 0;
     st->worst_err = 0u;
@@ -48,6 +47,15 @@ __global__ void k_pci_stats_reset(PciStatus* st0) {
     st->last_err = 0u;
     st->final_iter = -1;
   }
+}
+
+__global__ void k_pci_stats_reset(PciStatus* st0) { pci_reset_stats(st0 + blockIdx.x); }
+
+__global__ void k_pci_begin(PciStatus* st, ErrSlots es, uint32_t* flags, uint32_t* grid_flags) {
+  pci_reset_stats(st);
+  pci_reset_scene(st, 0, nullptr, es);
+  if (threadIdx.x < 2) flags[threadIdx.x] = 0u;
+  if (threadIdx.x == 2 && grid_flags) *grid_flags = 0u;
 }
 
 // The config-mode pair sums of the non-pressure pass in one walk over
@@ -524,6 +532,13 @@ psb_status launch_pci_retry_reset(PciStatus* st, hipStream_t s, ErrSlots es,
   return PSB_OK;
 }
 
+psb_status launch_pci_begin(PciStatus* st, ErrSlots es, uint32_t* flags, uint32_t* grid_flags,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(k_pci_begin, dim3(1), dim3(256), 0, s, st, es, flags, grid_flags);
+  PSB_HIP(hipGetLastError());
+  return PSB_OK;
+}
+
 psb_status launch_pci_reset(PciStatus* st, bool stats, hipStream_t s, uint32_t scenes,
                             uint32_t* done, ErrSlots es) {
   if (stats) hipLaunchKernelGGL(k_pci_stats_reset, dim3(scenes), dim3(64), 0, s, st);
@@ -802,11 +817,10 @@ static psb_status pci_sph_update_on(psb_context ctx, const psb_sph_params* prm, 
   b.aid = nullptr;
   const bool ref = prm->mode == PSB_MODE_REFERENCE;
   const bool warm = !ref && prm->warm_start == PSB_WARM_PREVIOUS;
-  PSB_HIP(hipMemsetAsync(ctx->d_flags, 0, 4, s));
   // start density (PciSphSystem.cu:17), scratch copies with v.w = 1/rho
   PSB_TRY(launch_density_list(n, c, nb, reinterpret_cast<const float4*>(pos4),
-                              reinterpret_cast<const float4*>(vel4), density, tmp_p, xs, vs, s));
-  if (!warm) PSB_HIP(hipMemsetAsync(pressure, 0, 4 * (size_t)n, s));
+                              reinterpret_cast<const float4*>(vel4), density, tmp_p, xs, vs,
+                              warm ? nullptr : pressure, s));
   // the start pressure is not read again: its n words hold the error slots
   // (with one word for all workgroups' maxima the density pass took 23.4 us
   // at 253,952 particles, now 18.2; 11.1 at 44,000, now 7.9)
@@ -815,7 +829,7 @@ static psb_status pci_sph_update_on(psb_context ctx, const psb_sph_params* prm, 
     es.base = reinterpret_cast<uint32_t*>(tmp_p);
     es.stride = n / kErrSlots;
   }
-  PSB_TRY(launch_pci_reset(st, true, s, 1, nullptr, es));
+  PSB_TRY(launch_pci_begin(st, es, ctx->d_flags, nullptr, s));
   PciOut o{};
   o.normals = reinterpret_cast<float4*>(normals4);
   o.fV = reinterpret_cast<float4*>(f_viscosity4);
@@ -854,12 +868,14 @@ static psb_status pci_sph_update_on(psb_context ctx, const psb_sph_params* prm, 
                              0, o, s, lanes));
     std::swap(cur, nxt);
     if (k + 1 >= c.min_it) {
-      PSB_HIP(hipMemcpyAsync(ctx->h_pinned, st, 16, hipMemcpyDeviceToHost, s));
+      PSB_TRY(launch_words_out(reinterpret_cast<const uint32_t*>(st), 4, nullptr, 0, nullptr, 0,
+                               ctx->d_pinned, s));
       PSB_HIP(hipStreamSynchronize(s));
-      const PciStatus* hs = reinterpret_cast<const PciStatus*>(ctx->h_pinned);
-      if (hs->final_iter >= 0) {
-        iters = hs->last_iters;
-        std::memcpy(&err, &hs->last_err, 4);
+      PciStatus hs;
+      std::memcpy(&hs, ctx->h_pinned, 16);
+      if (hs.final_iter >= 0) {
+        iters = hs.last_iters;
+        std::memcpy(&err, &hs.last_err, 4);
         break;
       }
     }

@@ -1049,7 +1049,8 @@ struct psb_context_s {
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
   uint32_t* d_flags = nullptr;     // device u32 flags for standalone calls
-  uint32_t* h_pinned = nullptr;    // pinned host staging (4 KiB)
+  uint32_t* h_pinned = nullptr;    // pinned, device-mapped host staging (4 KiB)
+  uint32_t* d_pinned = nullptr;    // its device address
 };
 
 struct psb_grid_s {
@@ -1073,6 +1074,11 @@ struct psb_grid_s {
 namespace psb {
 
 psb_status ensure_scratch(psb_context ctx, size_t bytes);
+// Up to three short device arrays, one after another, into device-mapped host
+// memory by one kernel (a few status words: one copy each is a launch of ~4 us
+// apiece, staged through pageable memory where the target is that).
+psb_status launch_words_out(const uint32_t* a, uint32_t na, const uint32_t* b, uint32_t nb,
+                            const uint32_t* c, uint32_t nc, uint32_t* out, hipStream_t s);
 GridDev grid_dev(const psb_grid_desc& d, float h);
 
 // Particle state arrays moved by the stable reorder (src -> dst[rank]).

@@ -35,6 +35,22 @@ psb_status hip_fail(hipError_t e, const char* what, const char* file, int line) 
   return PSB_ERR_HIP;
 }
 
+__global__ void k_words_out(const uint32_t* a, uint32_t na, const uint32_t* b, uint32_t nb,
+                            const uint32_t* c, uint32_t nc, uint32_t* out) {
+  const uint32_t t = threadIdx.x;
+  if (t < na) out[t] = a[t];
+  else if (t < na + nb) out[t] = b[t - na];
+  else if (t < na + nb + nc) out[t] = c[t - na - nb];
+}
+
+psb_status launch_words_out(const uint32_t* a, uint32_t na, const uint32_t* b, uint32_t nb,
+                            const uint32_t* c, uint32_t nc, uint32_t* out, hipStream_t s) {
+  PSB_ARG(na + nb + nc <= 64, "too many words");
+  hipLaunchKernelGGL(k_words_out, dim3(1), dim3(64), 0, s, a, na, b, nb, c, nc, out);
+  PSB_HIP(hipGetLastError());
+  return PSB_OK;
+}
+
 psb_status ensure_scratch(psb_context ctx, size_t bytes) {
   if (ctx->scratch_bytes >= bytes) return PSB_OK;
   if (ctx->scratch) PSB_HIP(hipFree(ctx->scratch));
@@ -306,7 +322,9 @@ psb_status psb_init(int32_t device, psb_context* out) {
   hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
   if (e != hipSuccess) { delete ctx; return hip_fail(e, "hipStreamCreate", __FILE__, __LINE__); }
   e = hipMalloc(&ctx->d_flags, 64);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&ctx->h_pinned, 4096, hipHostMallocDefault);
+  if (e == hipSuccess)
+    e = hipHostMalloc((void**)&ctx->h_pinned, 4096, hipHostMallocMapped | hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&ctx->d_pinned, ctx->h_pinned, 0);
   if (e != hipSuccess) { psb_finalize(ctx); return hip_fail(e, "context buffers", __FILE__, __LINE__); }
   // device address of this GPU's copy of the allocation-free entry point's
   // static scratch (psb_pci_sph_update_noalloc)

@@ -30,9 +30,11 @@ __global__ __launch_bounds__(256) void k_density_list(uint32_t n, Consts c,
                                                       float* __restrict__ rho,
                                                       float* __restrict__ pres,
                                                       float4* __restrict__ xs,
-                                                      float4* __restrict__ vs) {
+                                                      float4* __restrict__ vs,
+                                                      float* __restrict__ zero) {
   const uint32_t p = particle_index();
   if (p >= n) return;
+  if (zero) zero[p] = 0.f;
   const float4 xi = pos[p];
   float S = 0.f;
   const uint32_t m = cnt[p];
@@ -186,10 +188,10 @@ __global__ __launch_bounds__(256) void k_collider(uint32_t n, ColliderDev k, flo
 // ---- launchers used by system.hip --------------------------------------------
 psb_status launch_density_list(uint32_t n, const Consts& c, psb_neighbors nb, const float4* pos,
                                const float4* vel, float* rho, float* pres, float4* xs, float4* vs,
-                               hipStream_t s) {
+                               float* zero, hipStream_t s) {
   if (!n) return PSB_OK;
   hipLaunchKernelGGL(k_density_list, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, c, nb.count,
-                     nb.list, pos, vel, rho, pres, xs, vs);
+                     nb.list, pos, vel, rho, pres, xs, vs, zero);
   PSB_HIP(hipGetLastError());
   return PSB_OK;
 }
@@ -246,7 +248,8 @@ psb_status psb_evaluate_densities_forces(psb_context ctx, const psb_sph_params* 
   float4* vs = xs + n;
   hipLaunchKernelGGL(k_density_list, dim3(blocks_for(n)), dim3(kBlock), 0, ctx->stream, n, c,
                      nb.count, nb.list, reinterpret_cast<const float4*>(pos4),
-                     reinterpret_cast<const float4*>(vel4), density, pressure, xs, vs);
+                     reinterpret_cast<const float4*>(vel4), density, pressure, xs, vs,
+                     (float*)nullptr);
   WcsphOut o{};
   o.normals = reinterpret_cast<float4*>(normals4);
   o.fP = reinterpret_cast<float4*>(f_pressure4);
