@@ -227,6 +227,53 @@ __global__ __launch_bounds__(256) void k_rank_reorder(const uint32_t* __restrict
   }
 }
 
+// End of a particle's search: count, density (with the epilogue fused), flags.
+// (x.w written by the epilogue is not read by the search: it tests positions
+// only.)
+template <bool DENS, class M>
+__device__ __forceinline__ void search_finish(const M& map, uint32_t p, uint32_t sc, uint32_t n,
+                                              uint32_t cnt, uint32_t cap, bool wide, float S,
+                                              uint32_t* __restrict__ ncount,
+                                              float* __restrict__ rho, float mc,
+                                              uint32_t* __restrict__ flags, const Compact16& c16,
+                                              const EpiArgs& ep) {
+  ncount[p] = cnt < cap ? cnt : cap;
+  if (DENS) {
+    if (ep.on) {
+      Consts cc = ep.c;
+      map.patch(cc, sc);
+      density_epilogue_one(cc, ep, p, S * mc, rho);
+    } else {
+      rho[p] = S * mc;
+    }
+  }
+  if (cnt > cap) atomicOr(flags, PSB_FLAG_NEIGHBOR_OVERFLOW);
+  if (wide) atomicOr(c16.wide + (size_t)sc * c16.wide_stride, 1u);
+}
+
+// Workgroup maximum of the neighbour counts, then one atomic per workgroup on
+// a spread slot (every thread of the workgroup calls it).
+template <class M>
+__device__ __forceinline__ void report_max_count(const M& map, uint32_t cnt,
+                                                 uint32_t* __restrict__ maxcnt, ErrSlots es) {
+  if (!maxcnt && !es.base) return;
+  __shared__ uint32_t red[8];
+  const uint32_t m = wave_max_u(cnt);
+  if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t b = 0;
+    for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) b = max(b, red[w]);
+    if (b) {
+      uint32_t* dst = es.base ? es.base + (size_t)(blockIdx.x % kErrSlots) * es.stride +
+                                    (size_t)map.scene_of_block() * kMaxIterSlots + kCountEntry
+                              : maxcnt;
+      // most workgroups find a maximum no smaller than theirs already there
+      if (b > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, b);
+    }
+  }
+}
+
 // searchNeighbooring (UniformGridKernel.cu:58-95) on sorted positions; the
 // density sum of the same pairs rides along (SphKernel.cu:9-27).
 // RT > 0: the stencil half-width is a compile-time constant; the (2RT+1)^2
@@ -337,38 +384,237 @@ __global__ __launch_bounds__(M::kMaxThreads) void k_neighbors(M map, const float
         }
       }
     }
-    ncount[p] = cnt < cap ? cnt : cap;
-    if (DENS) {
-      if (ep.on) {
-        // the density epilogue, fused (x.w written here is not read by the
-        // search: it tests positions only)
-        Consts cc = ep.c;
-        map.patch(cc, sc);
-        density_epilogue_one(cc, ep, p, S * mc, rho);
+    search_finish<DENS>(map, p, sc, n, cnt, cap, wide, S, ncount, rho, mc, flags, c16, ep);
+  }
+  report_max_count(map, cnt, maxcnt, es);
+}
+
+// The same search for few particles: a workgroup of kSplit waves serves 64
+// particles, each lane a contiguous kPer of the (2 RT + 1)^2 stencil rows of
+// one particle.  With a lane per particle the search is a serial chain of
+// ~6,000 instructions however few the particles are; here a particle's tests
+// run side by side, and what is left in sequence is the density sum over its
+// neighbours' weights.
+//
+// Every lane keeps its accepted candidates (index less the particle's) in
+// LDS.  The counts of a particle's lanes, in row order, place them in the
+// list; the waves take eight of a particle's entries each, write them (whole
+// words of the compact list, rows of 64 in the plain one) and leave their
+// weights in LDS, which the first wave adds in list order: list and sum are
+// the plain search's.  40 KB a workgroup, so that four fit a compute unit.
+// Where a buffer does not hold all (more accepted candidates, or an index too
+// far away), the particle's lanes write their own entries, and the lane of
+// that buffer walks its rows again.
+// Bound by latency at 1,000 particles (with the density sum 9.0 us, a lane
+// per particle 30), by instruction issue at 100,000 (27 us against 35).
+constexpr int kSplit = 5;             // lanes per particle
+constexpr uint32_t kSplitHits = 44;   // accepted candidates kept per lane
+constexpr uint32_t kSplitSum = 40;    // weights kept per particle (a multiple of 8)
+// Candidate loads in flight per stencil row (an earlier form: 6 13.7 us at
+// 32,768 particles, 8 14.5, 6 without those past the row's end 14.3).
+constexpr int kSplitSlots = 6;
+template <int RT> struct SplitShape {
+  static constexpr int kWidth = 2 * RT + 1;
+  static constexpr int kRows = kWidth * kWidth;
+  static constexpr int kPer = (kRows + kSplit - 1) / kSplit;   // rows per lane
+};
+
+template <bool DENS, int RT>
+__global__ __launch_bounds__(64 * kSplit) void k_neighbors_split(
+    const float4* xs, uint32_t n, GridDev g, const uint32_t* __restrict__ start, float r2,
+    uint32_t cap, uint32_t* __restrict__ ncount, uint32_t* __restrict__ nlist,
+    float* __restrict__ rho, float mc, uint32_t* __restrict__ flags, uint32_t* __restrict__ maxcnt,
+    Compact16 c16, ErrSlots es, EpiArgs ep) {
+  using Sh = SplitShape<RT>;
+  constexpr int W = Sh::kWidth, kPer = Sh::kPer;
+  constexpr uint32_t kOver = 0x80000000u;   // flag in count: the lane's buffer does not hold all
+  constexpr uint32_t kPitch = kSplitHits + 1;   // one more takes what does not fit
+  __shared__ int16_t rel[kSplit * kPitch * 64];
+  __shared__ float weight[DENS ? kSplitSum * 64 : 1];
+  __shared__ uint32_t count[kSplit][64];
+  const uint32_t i = threadIdx.x & 63u;
+  const uint32_t slice = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t p = xcd_block(blockIdx.x, gridDim.x) * 64u + i;
+  const bool valid = p < n;
+  uint32_t q0[kPer] = {}, q1[kPer] = {}, c = 0, cnt = 0;
+  float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
+  int cx = 0, cy = 0, cz = 0;
+  bool over = false;
+  auto range = [&](int r, uint32_t& lo, uint32_t& hi) {
+    const int z = cz + r / W - RT, y = cy + r % W - RT;
+    const bool in = r < Sh::kRows && z >= 0 && z < g.nz && y >= 0 && y < g.ny;
+    const uint64_t base = in ? (uint64_t)g.nx * ((uint64_t)y + (uint64_t)g.ny * (uint64_t)z) : 0;
+    lo = start[base + max(cx - RT, 0)];
+    hi = start[base + min(cx + RT, g.nx - 1) + 1];
+    if (!in) hi = lo;
+  };
+  auto weight_of = [&](const float4& xj, bool& acc) {
+    const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+    const float d2 = dot3(dx, dy, dz, dx, dy, dz);
+    acc = d2 <= r2;
+    return r2 - d2;
+  };
+  if (valid) {
+    xi = xs[p];
+    uint32_t bad = 0;
+    cx = cell_coord(xi.x, g.minx, g.cell, g.nx, bad);
+    cy = cell_coord(xi.y, g.miny, g.cell, g.ny, bad);
+    cz = cell_coord(xi.z, g.minz, g.cell, g.nz, bad);
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) range((int)slice * kPer + r, q0[r], q1[r]);
+    // one round of kSplitSlots candidates (loads past the row's end stay inside
+    // the array and are not accepted)
+    auto load = [&](uint32_t q, float4 (&xq)[kSplitSlots]) {
+#pragma unroll
+      for (int u = 0; u < kSplitSlots; ++u) xq[u] = gather4(xs, min(q + u, n - 1u));
+    };
+    // candidates from q on, the row's last `left`
+    const uint32_t mine = slice * kPitch * 64u + i;
+    auto test = [&](uint32_t q, uint32_t left, const float4 (&xq)[kSplitSlots]) {
+      // offsets of a round reach at most kSplitSlots past its first
+      const int d = (int)(q - p);
+      over = over || d < -kCompactReach || d > kCompactReach - kSplitSlots;
+#pragma unroll
+      for (int u = 0; u < kSplitSlots; ++u) {
+        bool acc;
+        weight_of(xq[u], acc);
+        rel[mine + 64u * min(c, kSplitHits)] = (int16_t)(d + u);
+        c += acc && (uint32_t)u < left ? 1u : 0u;
+      }
+    };
+    // the next row's first round loaded before this row's tests
+    float4 x0[2][kSplitSlots];
+    load(q0[0], x0[0]);
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      if (r + 1 < kPer) load(q0[r + 1], x0[(r + 1) & 1]);
+      if (q0[r] == q1[r]) continue;
+      test(q0[r], q1[r] - q0[r], x0[r & 1]);
+      for (uint32_t q = q0[r] + kSplitSlots; q < q1[r]; q += kSplitSlots) {
+        float4 xq[kSplitSlots];
+        load(q, xq);
+        test(q, q1[r] - q, xq);
+      }
+    }
+    over = over || c > kSplitHits;
+    count[slice][i] = c | (over ? kOver : 0u);
+  }
+  __syncthreads();
+  bool wide = false, listed = true;   // listed: every buffer of the particle holds all
+  uint32_t end[kSplit] = {}, at = 0, all = 0;
+  // entry k of the particle's list, less p
+  auto entry = [&](uint32_t k) {
+    uint32_t e = k;
+#pragma unroll
+    for (uint32_t s = 1; s < (uint32_t)kSplit; ++s)
+      e = k >= end[s - 1] ? s * kPitch + k - end[s - 1] : e;
+    return (int)rel[e * 64u + i];
+  };
+  if (valid) {
+#pragma unroll
+    for (uint32_t s = 0; s < (uint32_t)kSplit; ++s) {
+      const uint32_t m = count[s][i];
+      listed = listed && !(m & kOver);
+      at = s == slice ? all : at;
+      all += m & ~kOver;
+      end[s] = all;
+    }
+    uint32_t* const l32g = (c16.list32g && c16.want32 && *c16.want32) ? c16.list32g : nullptr;
+    if (listed) {
+      for (uint32_t k0 = 8u * slice; k0 < (DENS ? all : min(all, cap)); k0 += 8u * kSplit) {
+        int d[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) d[u] = entry(min(k0 + u, all - 1u));
+        if (DENS && k0 < kSplitSum) {
+          float4 xq[8];
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u) xq[u] = gather4(xs, p + (uint32_t)d[u]);
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u) {
+            bool acc;
+            weight[(k0 + u) * 64u + i] = weight_of(xq[u], acc);
+          }
+        }
+        if (k0 >= cap) continue;
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u)
+          if (k0 + u < min(all, cap)) nlist[(uint64_t)(k0 + u) * n + p] = p + (uint32_t)d[u];
+        if (l32g) {
+          uint4* const dst = reinterpret_cast<uint4*>(l32g + l32g_at(k0, p, n));
+          dst[0] = make_uint4(p + d[0], p + d[1], p + d[2], p + d[3]);
+          dst[n] = make_uint4(p + d[4], p + d[5], p + d[6], p + d[7]);
+        } else if (c16.list16) {
+          uint32_t v[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            v[u] = (uint32_t)(d[2 * u] + 32768) | (uint32_t)(d[2 * u + 1] + 32768) << 16;
+          *reinterpret_cast<uint4*>(c16.list16 + l16_at(k0, p, n)) = make_uint4(v[0], v[1], v[2], v[3]);
+        }
+      }
+    } else {
+      auto put = [&](uint32_t k, uint32_t q) {
+        if (k >= cap) return;
+        nlist[(uint64_t)k * n + p] = q;
+        if (l32g) l32g[l32g_at(k, p, n)] = q;
+        else if (c16.list16) {
+          const int d = (int)(q - p);
+          const bool fits = d >= -kCompactReach && d <= kCompactReach;
+          if (fits) c16.list16[l16_at(k, p, n)] = (uint16_t)(d + 32768);
+          wide = wide || !fits;
+        }
+      };
+      if (!over) {
+        for (uint32_t k = 0; k < c; ++k) put(at + k, p + (int)rel[(slice * kPitch + k) * 64u + i]);
       } else {
-        rho[p] = S * mc;
+#pragma unroll
+        for (int r = 0; r < kPer; ++r)
+          for (uint32_t q = q0[r]; q < q1[r]; ++q) {
+            bool acc;
+            weight_of(gather4(xs, q), acc);
+            if (acc) put(at++, q);
+          }
       }
     }
-    if (cnt > cap) atomicOr(flags, PSB_FLAG_NEIGHBOR_OVERFLOW);
-    if (wide) atomicOr(c16.wide + (size_t)sc * c16.wide_stride, 1u);
+    if (wide && slice != 0u) atomicOr(c16.wide, 1u);
   }
-  if (maxcnt || es.base) {
-    // workgroup maximum, then one atomic per workgroup on a spread slot
-    __shared__ uint32_t red[M::kMaxThreads / 64];
-    const uint32_t m = wave_max_u(cnt);
-    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t b = 0;
-      for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) b = max(b, red[w]);
-      if (b) {
-        uint32_t* dst = es.base ? es.base + (size_t)(blockIdx.x % kErrSlots) * es.stride +
-                                      (size_t)map.scene_of_block() * kMaxIterSlots + kCountEntry
-                                : maxcnt;
-        atomicMax(dst, b);
+  if (DENS) __syncthreads();
+  if (valid && slice == 0u) {
+    cnt = all;
+    float S = 0.f;
+    if (DENS && listed) {
+      for (uint32_t k = 0; k < min(all, kSplitSum); k += 8u) {
+        float w[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) w[u] = weight[(k + u) * 64u + i];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u)
+          if (k + u < all) S = __builtin_fmaf(w[u] * w[u], w[u], S);
+      }
+      for (uint32_t k = kSplitSum; k < all; k += 8u) {
+        float4 xq[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) xq[u] = gather4(xs, p + entry(min(k + u, all - 1u)));
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+          bool acc;
+          const float w = weight_of(xq[u], acc);
+          if (k + u < all) S = __builtin_fmaf(w * w, w, S);
+        }
+      }
+    } else if (DENS) {
+      for (int r = 0; r < Sh::kRows; ++r) {
+        uint32_t lo, hi;
+        range(r, lo, hi);
+        for (uint32_t q = lo; q < hi; ++q) {
+          bool acc;
+          const float w = weight_of(gather4(xs, q), acc);
+          if (acc) S = __builtin_fmaf(w * w, w, S);
+        }
       }
     }
+    search_finish<DENS>(SingleMap{}, p, 0u, n, cnt, cap, wide, S, ncount, rho, mc, flags, c16, ep);
   }
+  report_max_count(SingleMap{}, cnt, maxcnt, es);
 }
 
 template <int W>
@@ -582,6 +828,29 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   dim3 gb(blocks_for(n)), tb(kBlock);
   EpiArgs e{};
   if (ep && rho) e = *ep;
+  // Several lanes per particle, for the stencils that have that kernel; with
+  // the density sum while one lane leaves the chip short of waves.  Us, one
+  // lane -> kSplit, jittered lattices, cells of half the radius:
+  //   without the sum    1,000 25.0 -> 6.1   32,768 24.7 -> 8.1   97,336 29.1
+  //                      -> 16.9  253,952 36.6 -> 32.9  474,552 65.0 -> 53.2
+  //   with it            4,096 30.5 -> 9.0   32,768 30.2 -> 12.4  97,336 34.6
+  //                      -> 27.3  157,464 39.0 -> 37.4  195,112 40.8 -> 44.5
+  // (cells of the radius: 32,768 31.9 -> 10.9 and 34.3 -> 13.4, 110,592 39.2
+  // -> 23.6 and 40.9 -> 31.8, 262,144 58.7 -> 45.4 and 59.0 -> 66.0).  Staged
+  // tiles keep the plain search.
+  int cus = 0;
+  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->ctx->device));
+  if (!tiles && (R == 1 || R == 2) && (!rho || n <= 576ull * (uint64_t)cus)) {
+#define PSB_NBS(D_, R_)                                                                           \
+  hipLaunchKernelGGL((k_neighbors_split<D_, R_>), dim3(blocks_for(n, 64u)),                       \
+                     dim3(64 * kSplit), 0, s, xs, n, gd, g->start, r2, nb.capacity, \
+                     nb.count, nb.list, rho, mc, flags, maxcnt, c16, es, e)
+    if (rho) { if (R == 1) PSB_NBS(true, 1); else PSB_NBS(true, 2); }
+    else { if (R == 1) PSB_NBS(false, 1); else PSB_NBS(false, 2); }
+#undef PSB_NBS
+    PSB_HIP(hipGetLastError());
+    return PSB_OK;
+  }
 #define PSB_NB(D_, R_)                                                                       \
   hipLaunchKernelGGL((k_neighbors<D_, R_, SingleMap>), gb, tb, 0, s, SingleMap{}, xs, n, gd,    \
                      g->start, r2, nb.capacity, nb.count, nb.list, rho, mc, flags, maxcnt, c16, es, \
@@ -589,7 +858,7 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   if (rho) {
     if (R == 1) PSB_NB(true, 1); else if (R == 2) PSB_NB(true, 2); else PSB_NB(true, 0);
   } else {
-    if (R == 1) PSB_NB(false, 1); else if (R == 2) PSB_NB(false, 2); else PSB_NB(false, 0);
+    PSB_NB(false, 0);
   }
 #undef PSB_NB
   PSB_HIP(hipGetLastError());
@@ -721,7 +990,7 @@ psb_status psb_search_neighbors(psb_grid g, const float* sorted_pos4, uint32_t n
   PSB_HIP(hipMemsetAsync(ctx->d_flags, 0, 8, ctx->stream));
   GridDev gd = grid_dev(g->desc, radius);
   PSB_TRY(launch_neighbors(g, reinterpret_cast<const float4*>(sorted_pos4), n, radius * radius,
-                           gd.R, nb, nullptr, 0.f, ctx->d_flags, ctx->d_flags + 1, ctx->stream));
+                           gd.R, nb, nullptr, 0.f, ctx->d_flags, nullptr, ctx->stream));
   PSB_TRY(launch_words_out(ctx->d_flags, 2, g->flags, 1, nullptr, 0, ctx->d_pinned, ctx->stream));
   PSB_HIP(hipStreamSynchronize(ctx->stream));
   if (flags_out) *flags_out = ctx->h_pinned[0] | ctx->h_pinned[2];
