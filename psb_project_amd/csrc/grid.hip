@@ -11,7 +11,7 @@
 //   2. k_scan_*       start = exclusive prefix sum of count over all cells
 //                     (start[c] = #particles with hash < c, start[ncells] = n);
 //                     the per-tile sums come from step 1 (tsum), so the scan
-//                     reads count once; k_rank_reorder re-zeroes the occupied
+//                     reads count once, and only where particles are; k_rank_reorder re-zeroes the occupied
 //                     cells' counts for the next build
 //   3. k_scatter      tmp[start[c] + slot[i]] = i      (order within a cell
 //                     still depends on the atomics)
@@ -29,6 +29,13 @@ namespace psb {
 
 constexpr int kTileSlots = 16;   // copies of the per-tile count table (atomic spreading)
 
+// Bound by its atomics: one per run of lanes in the same cell and, where the
+// scan's tiles fit in LDS, one per workgroup and tile (43,993 particles in
+// random order 10.9 -> 6.0 us, where a wave went through up to 64 tiles in
+// turn; 262,144 in cells of eight 27.3 -> 7.8).  Larger tables are counted by
+// wave: a workgroup would pay more to clear and send the table.
+constexpr uint32_t kLdsTiles = 512;   // scan tiles counted in LDS
+
 // M: SingleMap or BatchMap (a batch hashes into its scene's cell range).
 template <class M>
 __global__ __launch_bounds__(M::kMaxThreads) void k_hash_count(M map, const float4* __restrict__ pos,
@@ -40,26 +47,52 @@ __global__ __launch_bounds__(M::kMaxThreads) void k_hash_count(M map, const floa
                                                                uint32_t* __restrict__ tsum,
                                                                uint32_t nscan, StepReset rs) {
   if (rs.st && blockIdx.x < rs.scenes) pci_reset_scene(rs.st, blockIdx.x, rs.done, rs.es);
-  uint32_t i, sc;
+  __shared__ uint32_t tiles[kLdsTiles];
+  if (nscan <= kLdsTiles) {
+    for (uint32_t t = threadIdx.x; t < nscan; t += blockDim.x) tiles[t] = 0u;
+    __syncthreads();
+  }
+  uint32_t i = 0, sc = 0, off = 0, c = 0xFFFFFFFFu, bad = 0, f = 0;
   bool lead;
-  if (!map.locate(n, i, sc, lead)) return;
-  uint32_t off;
-  const GridDev g = map.grid(g0, sc, off);
-  float4 p = pos[i];
-  uint32_t bad = 0;
-  int cx = cell_coord(p.x, g.minx, g.cell, g.nx, bad);
-  int cy = cell_coord(p.y, g.miny, g.cell, g.ny, bad);
-  int cz = cell_coord(p.z, g.minz, g.cell, g.nz, bad);
-  uint32_t c = off + (uint32_t)cx + (uint32_t)g.nx * ((uint32_t)cy + (uint32_t)g.ny * (uint32_t)cz);
-  hash[i] = c;
-  slot[i] = atomicAdd(&count[c], 1u);
-  // per-scan-tile particle counts (the scan's first pass), one atomic per
-  // distinct tile of the wave (the particles arrive in last step's sorted
-  // order, so a wave's cells mostly share a tile), spread over kTileSlots
-  // copies of the table by workgroup
+  const bool valid = map.locate(n, i, sc, lead);
+  if (valid) {
+    const GridDev g = map.grid(g0, sc, off);
+    const float4 p = pos[i];
+    const int cx = cell_coord(p.x, g.minx, g.cell, g.nx, bad);
+    const int cy = cell_coord(p.y, g.miny, g.cell, g.ny, bad);
+    const int cz = cell_coord(p.z, g.minz, g.cell, g.nz, bad);
+    c = off + (uint32_t)cx + (uint32_t)g.nx * ((uint32_t)cy + (uint32_t)g.ny * (uint32_t)cz);
+    hash[i] = c;
+    if (bad) f |= PSB_FLAG_OUT_OF_GRID;
+    if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z))) f |= PSB_FLAG_NONFINITE;
+    if (f) atomicOr(flags, f);
+  }
+  // one atomic per run of lanes in the same cell (a cell's slots are given out
+  // in any order; atomics on one cell's word serialise)
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t prev = (uint32_t)__shfl_up((int)c, 1, 64);
+  const uint64_t heads = __ballot(lane == 0u || c != prev);
+  const uint32_t head = 63u - (uint32_t)__builtin_clzll(heads & (~0ull >> (63u - lane)));
+  const uint64_t later = lane == 63u ? 0ull : heads >> (lane + 1u);
+  const uint32_t run = later ? (uint32_t)__builtin_ctzll(later) + 1u : 64u - lane;
+  uint32_t first = 0;
+  if (valid && head == lane) first = atomicAdd(&count[c], run);
+  first = (uint32_t)__shfl((int)first, (int)head, 64);
+  if (valid) slot[i] = first + lane - head;
+  // per-scan-tile particle counts (the scan's first pass), spread over
+  // kTileSlots copies of the table by workgroup: counted in LDS where the
+  // table fits, else one atomic per distinct tile of the wave (the particles
+  // arrive in last step's sorted order, so a wave's cells mostly share a tile)
   const uint32_t t = c / kScanTile;
   uint32_t* __restrict__ ts = tsum + (size_t)(blockIdx.x % kTileSlots) * nscan;
-  uint64_t todo = __ballot(1);
+  if (nscan <= kLdsTiles) {
+    if (valid && head == lane) atomicAdd(&tiles[t], run);
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < nscan; k += blockDim.x)
+      if (tiles[k]) atomicAdd(&ts[k], tiles[k]);
+    return;
+  }
+  uint64_t todo = __ballot(valid);
   while (todo) {
     const int leader = __ffsll((unsigned long long)todo) - 1;
     const uint32_t tl = (uint32_t)__shfl((int)t, leader, 64);
@@ -67,13 +100,10 @@ __global__ __launch_bounds__(M::kMaxThreads) void k_hash_count(M map, const floa
     if ((int)(threadIdx.x & 63u) == leader) atomicAdd(&ts[tl], (uint32_t)__popcll(same));
     todo &= ~same;
   }
-  uint32_t f = 0;
-  if (bad) f |= PSB_FLAG_OUT_OF_GRID;
-  if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z))) f |= PSB_FLAG_NONFINITE;
-  if (f) atomicOr(flags, f);
 }
 
-// exclusive scan of one value per thread over a 256-thread block
+// exclusive scan of one value per thread over a workgroup of W waves
+template <uint32_t W = 4>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds, uint32_t& total) {
   const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
   uint32_t x = v;
@@ -86,7 +116,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds, u
   __syncthreads();
   uint32_t woff = 0, tot = 0;
 #pragma unroll
-  for (uint32_t w = 0; w < 4; ++w) {
+  for (uint32_t w = 0; w < W; ++w) {
     uint32_t t = lds[w];
     if (w < wid) woff += t;
     tot += t;
@@ -117,77 +147,127 @@ __global__ __launch_bounds__(256) void k_scan_reduce(const uint32_t* __restrict_
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-// exclusive scan of the tile sums in one workgroup: dst[k] = sum of src[<k]
-// (dst may be src).  CONSUME: src holds kTileSlots tables of nb partial sums
-// (added here) and is zeroed for the next build.  start[ncells] = total.
-template <bool CONSUME>
-__global__ __launch_bounds__(256) void k_scan_tiles(uint32_t* src, uint32_t* dst, uint32_t nb,
-                                                    uint32_t* __restrict__ start, uint64_t ncells) {
-  __shared__ uint32_t lds[4];
-  uint32_t carry = 0;
-  for (uint32_t b0 = 0; b0 < nb; b0 += 256) {
-    uint32_t k = b0 + threadIdx.x;
+// exclusive scan of the tile sums: dst[k] = sum of src[<k]; start[ncells] =
+// total.  PARTS: src holds kTileSlots tables of nb partial sums (added here),
+// dst is another array, and a workgroup takes kTilesPer tiles, adding up all
+// earlier ones itself: 37 -> 10.9 us at 8,192 tiles, where one workgroup of
+// 256 went through them a round trip to memory at a time.  Otherwise one
+// workgroup, and dst may be src.
+constexpr uint32_t kTilesPer = 1024;
+template <bool PARTS>
+__global__ __launch_bounds__(kTilesPer) void k_scan_tiles(const uint32_t* src, uint32_t* dst,
+                                                          uint32_t nb,
+                                                          uint32_t* __restrict__ start,
+                                                          uint64_t ncells) {
+  constexpr uint32_t W = kTilesPer / 64;
+  __shared__ uint32_t lds[W];
+  auto tile = [&](uint32_t k) {
+    if (!PARTS) return src[k];
     uint32_t v = 0u;
-    if (k < nb) {
-      if (CONSUME) {
 #pragma unroll
-        for (int j = 0; j < kTileSlots; ++j) {
-          v += src[(size_t)j * nb + k];
-          src[(size_t)j * nb + k] = 0u;
-        }
-      } else {
-        v = src[k];
-      }
-    }
-    uint32_t tot;
-    uint32_t ex = block_excl_scan(v, lds, tot);
+    for (int j = 0; j < kTileSlots; ++j) v += src[(size_t)j * nb + k];
+    return v;
+  };
+  const uint32_t b1 = PARTS ? min((blockIdx.x + 1u) * kTilesPer, nb) : nb;
+  uint32_t b0 = 0, carry = 0, tot;
+  if (PARTS && blockIdx.x) {
+    b0 = blockIdx.x * kTilesPer;
+    uint32_t v = 0;
+#pragma unroll 2
+    for (uint32_t k = threadIdx.x; k < b0; k += kTilesPer) v += tile(k);
+    block_excl_scan<W>(v, lds, carry);
+  }
+  for (; b0 < b1; b0 += kTilesPer) {
+    const uint32_t k = b0 + threadIdx.x;
+    const uint32_t ex = block_excl_scan<W>(k < nb ? tile(k) : 0u, lds, tot);
     if (k < nb) dst[k] = carry + ex;
     carry += tot;
   }
-  if (threadIdx.x == 0) start[ncells] = carry;
+  if (b1 == nb && threadIdx.x == 0) start[ncells] = carry;
 }
 
-// start[c] = tile offset + in-tile exclusive prefix; ZERO: count[c] = 0
+// start[c] = tile offset + in-tile exclusive prefix; ZERO: count[c] = 0;
+// parts: the tile's kTileSlots partial sums zeroed for the next build.  Bound
+// by the table's bytes: the counts of a tile without particles are not read,
+// and every access of a wave is one contiguous kilobyte (33.5 million cells,
+// a twentieth of their tiles occupied: 55 -> 34 us).
 template <bool ZERO>
 __global__ __launch_bounds__(256) void k_scan_apply(uint32_t* __restrict__ count, uint64_t ncells,
                                                     const uint32_t* __restrict__ bsum,
-                                                    uint32_t* __restrict__ start) {
-  __shared__ uint32_t lds[4];
+                                                    uint32_t* __restrict__ start,
+                                                    uint32_t* __restrict__ parts) {
+  constexpr int kSegs = 4;   // segments of 1,024 cells, four per thread
+  __shared__ uint32_t lds[kSegs][4];
+  const uint32_t nb = gridDim.x;
   const uint32_t toff = bsum[blockIdx.x];   // loaded with the counts, not after the block scan
-  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * 16;
-  uint32_t v[16];
+  const uint32_t tend = blockIdx.x + 1u < nb ? bsum[blockIdx.x + 1u] : start[ncells];
+  if (parts && threadIdx.x < (uint32_t)kTileSlots) parts[(size_t)threadIdx.x * nb + blockIdx.x] = 0u;
+  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * 4u;
   const bool full = (uint64_t)(blockIdx.x + 1) * kScanTile <= ncells;
-  if (full) {
-    const uint4* c4 = reinterpret_cast<const uint4*>(count + base);
+  uint4 v[kSegs] = {};
+  if (tend != toff) {   // the same for the whole workgroup
+    if (full) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      uint4 t = c4[j];
-      v[4 * j] = t.x; v[4 * j + 1] = t.y; v[4 * j + 2] = t.z; v[4 * j + 3] = t.w;
-    }
-  } else {
+      for (int j = 0; j < kSegs; ++j) v[j] = *reinterpret_cast<const uint4*>(count + base + 1024u * j);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = (base + j < ncells) ? count[base + j] : 0u;
-  }
-  uint32_t s = 0;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) { uint32_t t = v[j]; v[j] = s; s += t; }
-  uint32_t tot;
-  uint32_t off = block_excl_scan(s, lds, tot) + toff;
-  if (full) {
-    uint4* s4 = reinterpret_cast<uint4*>(start + base);
-    uint4* c4 = reinterpret_cast<uint4*>(count + base);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      s4[j] = make_uint4(v[4 * j] + off, v[4 * j + 1] + off, v[4 * j + 2] + off, v[4 * j + 3] + off);
-      if (ZERO) c4[j] = make_uint4(0u, 0u, 0u, 0u);
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-      if (base + j < ncells) {
-        start[base + j] = v[j] + off;
-        if (ZERO) count[base + j] = 0u;
+      for (int j = 0; j < kSegs; ++j) {
+        const uint64_t c = base + 1024u * j;
+        if (c < ncells) v[j].x = count[c];
+        if (c + 1 < ncells) v[j].y = count[c + 1];
+        if (c + 2 < ncells) v[j].z = count[c + 2];
+        if (c + 3 < ncells) v[j].w = count[c + 3];
       }
+    }
+    const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+    uint32_t x[kSegs];   // inclusive sums over the wave
+#pragma unroll
+    for (int j = 0; j < kSegs; ++j) x[j] = v[j].x + v[j].y + v[j].z + v[j].w;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+      for (int j = 0; j < kSegs; ++j) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x[j], o, 64);
+        if (lane >= (uint32_t)o) x[j] += y;
+      }
+    if (lane == 63u)
+#pragma unroll
+      for (int j = 0; j < kSegs; ++j) lds[j][wid] = x[j];
+    __syncthreads();
+    uint32_t before = toff;
+#pragma unroll
+    for (int j = 0; j < kSegs; ++j) {
+      uint32_t mine = before;
+#pragma unroll
+      for (uint32_t w = 0; w < 4u; ++w) {
+        if (w < wid) mine += lds[j][w];
+        before += lds[j][w];
+      }
+      const uint4 t = v[j];
+      v[j].x = mine + x[j] - (t.x + t.y + t.z + t.w);
+      v[j].y = v[j].x + t.x;
+      v[j].z = v[j].y + t.y;
+      v[j].w = v[j].z + t.z;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kSegs; ++j) v[j] = make_uint4(toff, toff, toff, toff);
+  }
+#pragma unroll
+  for (int j = 0; j < kSegs; ++j) {
+    const uint64_t c = base + 1024u * j;
+    if (full) {
+      *reinterpret_cast<uint4*>(start + c) = v[j];
+      if (ZERO && tend != toff) *reinterpret_cast<uint4*>(count + c) = make_uint4(0u, 0u, 0u, 0u);
+    } else {
+      const uint32_t e[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (c + u < ncells) {
+          start[c + u] = e[u];
+          if (ZERO) count[c + u] = 0u;
+        }
+    }
   }
 }
 
@@ -631,10 +711,10 @@ static psb_status grid_sort(psb_grid g, uint32_t n, const ReorderArrays* ra, hip
   // the tile sums came with the hashes (tsum); the scan's second pass
   // leaves count alone, the reorder re-zeroes the occupied cells
   const uint32_t nb = blocks_for(n);
-  hipLaunchKernelGGL(k_scan_tiles<true>, dim3(1), dim3(kBlock), 0, s, g->tsum, g->bsum, g->nscan,
-                     g->start, g->ncells);
+  hipLaunchKernelGGL(k_scan_tiles<true>, dim3(blocks_for(g->nscan, kTilesPer)), dim3(kTilesPer), 0,
+                     s, g->tsum, g->bsum, g->nscan, g->start, g->ncells);
   hipLaunchKernelGGL(k_scan_apply<false>, dim3(g->nscan), dim3(kBlock), 0, s, g->count, g->ncells,
-                     g->bsum, g->start);
+                     g->bsum, g->start, g->tsum);
   if (n) {
     hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(kBlock), 0, s, g->hash, g->slot, n, g->start, g->tmp);
     if (ra) {
@@ -756,8 +836,9 @@ psb_status scan_exclusive(uint32_t* count, uint64_t n, uint32_t* bsum, uint32_t*
                           hipStream_t s) {
   const uint32_t nt = (uint32_t)((n + kScanTile - 1) / kScanTile);
   if (nt) hipLaunchKernelGGL(k_scan_reduce, dim3(nt), dim3(kBlock), 0, s, count, n, bsum);
-  hipLaunchKernelGGL(k_scan_tiles<false>, dim3(1), dim3(kBlock), 0, s, bsum, bsum, nt, start, n);
-  if (nt) hipLaunchKernelGGL(k_scan_apply<true>, dim3(nt), dim3(kBlock), 0, s, count, n, bsum, start);
+  hipLaunchKernelGGL(k_scan_tiles<false>, dim3(1), dim3(kTilesPer), 0, s, bsum, bsum, nt, start, n);
+  if (nt) hipLaunchKernelGGL(k_scan_apply<true>, dim3(nt), dim3(kBlock), 0, s, count, n, bsum, start,
+                             (uint32_t*)nullptr);
   PSB_HIP(hipGetLastError());
   return PSB_OK;
 }
