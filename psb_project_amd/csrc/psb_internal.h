@@ -1026,6 +1026,13 @@ __device__ __forceinline__ float split_total(const float (&a)[2], uint32_t lane)
   return lane == 0 ? a[0] + other : other + a[0];
 }
 
+// Orders a wave's LDS writes before its later LDS reads by other lanes (the
+// hardware runs a wave's LDS operations in order; this keeps the compiler from
+// moving them).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 template <int N> __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int o = N / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, N));

@@ -76,17 +76,12 @@ struct WcsphOut {
   uint32_t* flags;
 };
 
-// internalForces (SphKernel.cu:32-91) [+ gravity, leapfrog, box, interpolation]
+// Particle p's force densities from its pair sums [+ gravity, leapfrog, box,
+// interpolation].
 template <bool SURF, bool STEP>
-__global__ __launch_bounds__(256) void k_wcsph_forces(uint32_t n, Consts c,
-                                                      const uint32_t* __restrict__ cnt,
-                                                      const uint32_t* __restrict__ list,
-                                                      const float4* __restrict__ xs,
-                                                      const float4* __restrict__ vs,
-                                                      const float* __restrict__ rho, WcsphOut o) {
-  const uint32_t p = particle_index();
-  if (p >= n) return;
-  PairSums s = internal_sums<true, SURF>(c, p, n, cnt, list, xs, vs);
+__device__ __forceinline__ void wcsph_finish(uint32_t p, const Consts& c, const PairSums& s,
+                                             const float4* __restrict__ xs,
+                                             const float* __restrict__ rho, const WcsphOut& o) {
   const float ri = rho[p];
   const float cpf = -(c.m * ri);
   float fP[3] = {s.fp[0] * cpf, s.fp[1] * cpf, s.fp[2] * cpf};
@@ -120,6 +115,117 @@ __global__ __launch_bounds__(256) void k_wcsph_forces(uint32_t n, Consts c,
   finish_particle(c, p, x, vh, va, x0, o.bx, o.bv, o.bvh);
   o.bid[p] = o.aid[p];
   o.bp[p] = o.pres[p];
+}
+
+// internalForces (SphKernel.cu:32-91) [+ the step]
+template <bool SURF, bool STEP>
+__global__ __launch_bounds__(256) void k_wcsph_forces(uint32_t n, Consts c,
+                                                      const uint32_t* __restrict__ cnt,
+                                                      const uint32_t* __restrict__ list,
+                                                      const float4* __restrict__ xs,
+                                                      const float4* __restrict__ vs,
+                                                      const float* __restrict__ rho, WcsphOut o) {
+  const uint32_t p = particle_index();
+  if (p >= n) return;
+  const PairSums s = internal_sums<true, SURF>(c, p, n, cnt, list, xs, vs);
+  wcsph_finish<SURF, STEP>(p, c, s, xs, rho, o);
+}
+
+// The same without surface tension for few particles, eight lanes to one: the
+// lanes take eight list entries at a time and leave each pair's factors in
+// LDS, then six of them add one component each over the eight in list order,
+// so the sums are the one-lane kernel's.  That one is a serial chain of ~1,000
+// instructions at any particle count; here a step of the chain is two LDS
+// reads and one multiply-add.  Bound by latency at 1,000 particles, by
+// instruction issue at 97,336, where the work done eight-fold (loads of list
+// and particle, round by round) has caught up.
+constexpr int kForceLanes = 8;
+constexpr uint32_t kForceP = 256 / kForceLanes;   // particles per workgroup
+template <bool STEP>
+__global__ __launch_bounds__(256) void k_wcsph_forces_lanes(uint32_t n, Consts c,
+                                                            const uint32_t* __restrict__ cnt,
+                                                            const uint32_t* __restrict__ list,
+                                                            const float4* __restrict__ xs,
+                                                            const float4* __restrict__ vs,
+                                                            const float* __restrict__ rho,
+                                                            WcsphOut o) {
+  constexpr uint32_t L = kForceLanes;
+  // a particle's 8 pairs: direction and pressure factor, velocity difference
+  // and viscosity factor; 8 words of padding keep the particles of a wave on
+  // different banks
+  __shared__ __align__(16) float pairs[kForceP][L * 8 + 8];
+  const uint32_t lane = threadIdx.x % L, slot = threadIdx.x / L;
+  const uint32_t p = xcd_block(blockIdx.x, gridDim.x) * kForceP + slot;
+  const uint32_t pc = min(p, n - 1u);
+  const uint32_t m = p < n ? cnt[p] : 0u;
+  const float4 xi = xs[pc], vi = vs[pc];
+  // entry k, the last one past the end (the particle itself without entries)
+  auto entry = [&](uint32_t k) {
+    return m ? list[(uint64_t)min(k, m - 1u) * n + p] : pc;
+  };
+  uint32_t q = entry(lane);
+  float4 xj = gather4(xs, q), vj = gather4(vs, q);
+  q = entry(lane + L);
+  float* const mine = pairs[slot];
+  const uint32_t ca = lane < 3u ? lane : lane + 1u;   // of lanes 0..5
+  const uint32_t cb = lane < 3u ? 3u : 7u;
+  float sum = 0.f;
+  for (uint32_t k0 = 0; __any(k0 < m); k0 += L) {
+    const float4 xn = gather4(xs, q), vn = gather4(vs, q);
+    q = entry(k0 + 2u * L + lane);
+    const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+    const float d2 = dot3(dx, dy, dz, dx, dy, dz);
+    // pairs that add nothing have all factors 0
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    if (d2 > 0.f && k0 + lane < m) {
+      float dd, invd;
+      dist_and_inverse(d2, dd, invd);
+      const float hd = c.h - dd;
+      const float gw = c.c_spiky * (hd * hd);
+      a = make_float4(dx * invd, dy * invd, dz * invd, gw * (xi.w + xj.w));
+      b = make_float4(vj.x - vi.x, vj.y - vi.y, vj.z - vi.z, hd * vj.w);
+    }
+    reinterpret_cast<float4*>(mine)[2u * lane] = a;
+    reinterpret_cast<float4*>(mine)[2u * lane + 1u] = b;
+    wave_lds_order();
+#pragma unroll
+    for (uint32_t e = 0; e < L; ++e)
+      sum = __builtin_fmaf(mine[8u * e + (ca & 7u)], mine[8u * e + cb], sum);
+    wave_lds_order();
+    xj = xn;
+    vj = vn;
+  }
+  PairSums s;
+  s.fs = s.nn[0] = s.nn[1] = s.nn[2] = 0.f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    s.fp[k] = __shfl(sum, k, kForceLanes);
+    s.fv[k] = __shfl(sum, k + 3, kForceLanes);
+  }
+  if (lane == 0u && p < n) wcsph_finish<false, STEP>(p, c, s, xs, rho, o);
+}
+
+// Launch of the force pass: eight lanes per particle up to 320 particles a
+// compute unit (one lane -> eight: 1,000 particles 10.3 -> 4.6 us, 32,768 12.5
+// -> 7.2, 46,656 12.9 -> 9.2, 64,000 13.2 -> 12.0; 97,336 15.8 -> 15.3).
+template <bool STEP>
+static psb_status launch_wcsph_forces(uint32_t n, const Consts& c, bool surf, const uint32_t* cnt,
+                                      const uint32_t* list, const float4* xs, const float4* vs,
+                                      const float* rho, const WcsphOut& o, hipStream_t s) {
+  int dev = 0, cus = 0;
+  PSB_HIP(hipGetDevice(&dev));
+  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  if (surf)
+    hipLaunchKernelGGL((k_wcsph_forces<true, STEP>), dim3(blocks_for(n)), dim3(kBlock), 0, s, n, c,
+                       cnt, list, xs, vs, rho, o);
+  else if (n <= 320ull * (uint64_t)cus)
+    hipLaunchKernelGGL((k_wcsph_forces_lanes<STEP>), dim3(blocks_for(n, kForceP)), dim3(256), 0, s,
+                       n, c, cnt, list, xs, vs, rho, o);
+  else
+    hipLaunchKernelGGL((k_wcsph_forces<false, STEP>), dim3(blocks_for(n)), dim3(kBlock), 0, s, n, c,
+                       cnt, list, xs, vs, rho, o);
+  PSB_HIP(hipGetLastError());
+  return PSB_OK;
 }
 
 // ---- pointwise kernels ------------------------------------------------------
@@ -215,14 +321,7 @@ psb_status launch_wcsph_step_forces(uint32_t n, const Consts& c, bool surf, cons
   WcsphOut o{};
   o.bx = bx; o.bv = bv; o.bvh = bvh; o.bid = bid; o.bp = bp; o.avh = avh; o.aid = aid;
   o.pres = pres; o.flags = flags;
-  if (surf)
-    hipLaunchKernelGGL((k_wcsph_forces<true, true>), dim3(blocks_for(n)), dim3(kBlock), 0, s, n, c,
-                       cnt, list, xs, vs, rho, o);
-  else
-    hipLaunchKernelGGL((k_wcsph_forces<false, true>), dim3(blocks_for(n)), dim3(kBlock), 0, s, n,
-                       c, cnt, list, xs, vs, rho, o);
-  PSB_HIP(hipGetLastError());
-  return PSB_OK;
+  return launch_wcsph_forces<true>(n, c, surf, cnt, list, xs, vs, rho, o, s);
 }
 
 }  // namespace psb
@@ -256,14 +355,9 @@ psb_status psb_evaluate_densities_forces(psb_context ctx, const psb_sph_params* 
   o.fV = reinterpret_cast<float4*>(f_viscosity4);
   o.fS = reinterpret_cast<float4*>(f_surface4);
   o.F = reinterpret_cast<float4*>(forces_accum4);
-  if (prm->surface_tension != 0.f)
-    hipLaunchKernelGGL((k_wcsph_forces<true, false>), dim3(blocks_for(n)), dim3(kBlock), 0,
-                       ctx->stream, n, c, nb.count, nb.list, xs, vs, density, o);
-  else
-    hipLaunchKernelGGL((k_wcsph_forces<false, false>), dim3(blocks_for(n)), dim3(kBlock), 0,
-                       ctx->stream, n, c, nb.count, nb.list, xs, vs, density, o);
   PSB_HIP(hipGetLastError());
-  return PSB_OK;
+  return launch_wcsph_forces<false>(n, c, prm->surface_tension != 0.f, nb.count, nb.list, xs, vs,
+                                    density, o, ctx->stream);
 }
 
 psb_status psb_force_constante(psb_context ctx, uint32_t n, float* accum4, const float* weight,
