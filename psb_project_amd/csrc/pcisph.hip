@@ -58,6 +58,22 @@ __global__ void k_pci_begin(PciStatus* st, ErrSlots es, uint32_t* flags, uint32_
   if (threadIdx.x == 2 && grid_flags) *grid_flags = 0u;
 }
 
+// The pressure scaling of a particle from its sums of gradients and of their
+// squares: the template delta, capped by 1/(beta (W1.W1 + W2)).
+__device__ __forceinline__ float np_delta(const Consts& c, const float4& xi, float W1x, float W1y,
+                                          float W1z, float W2) {
+  if (!c.delta_local_cap) return c.delta;
+  if (c.wall) {
+    // the static wall particles add to sum gradW, not to sum |gradW|^2
+    float S, wgx, wgy, wgz;
+    wall_sums<false, true>(c, xi.x, xi.y, xi.z, S, wgx, wgy, wgz);
+    W1x = W1x + wgx; W1y = W1y + wgy; W1z = W1z + wgz;
+  }
+  const float den = c.beta * (dot3(W1x, W1y, W1z, W1x, W1y, W1z) + W2);
+  const float loc = den > 0.f ? 1.0f / den : c.delta;
+  return loc < c.delta ? loc : c.delta;
+}
+
 // The config-mode pair sums of the non-pressure pass in one walk over
 // particle p's list: the viscosity (and surface) sums of internal_sums, and
 // the pressure scaling delta_i -- the template delta, capped by the
@@ -132,58 +148,19 @@ __device__ __forceinline__ PairSums np_sums(const Consts& c, uint32_t p, uint32_
     feat[6 * (size_t)n + p] = gy * c.h_over_ps;
     feat[7 * (size_t)n + p] = gz * c.h_over_ps;
   }
-  dl = c.delta;
-  if (!c.delta_local_cap) return s;
-  if (c.wall) {
-    // the static wall particles add to sum gradW, not to sum |gradW|^2
-    float S, wgx, wgy, wgz;
-    wall_sums<false, true>(c, xi.x, xi.y, xi.z, S, wgx, wgy, wgz);
-    W1x = W1x + wgx; W1y = W1y + wgy; W1z = W1z + wgz;
-  }
-  const float den = c.beta * (dot3(W1x, W1y, W1z, W1x, W1y, W1z) + W2);
-  if (den > 0.f) {
-    const float loc = 1.0f / den;
-    if (loc < c.delta) dl = loc;
-  }
+  dl = np_delta(c, xi, W1x, W1y, W1z, W2);
   return s;
 }
 
-// compute_Viscosity_SurfaceTension_Force_PCI (PciSphSystem_Kernel.cu:117-170)
-// + first prediction (integrateSPH_LeapFrog_Forces with f_P = 0).
-template <bool REF, bool SURF, bool WARM, bool OUT, bool FEAT, class M>
-__global__ __launch_bounds__(M::kMaxThreads) void k_pci_nonpressure(
-    M map, uint32_t n, Consts c, const uint32_t* __restrict__ cnt,
-    const uint32_t* __restrict__ list, const float4* __restrict__ xs,
-    const float4* __restrict__ vs, const float* __restrict__ rho, const float4* __restrict__ avh,
-    const float* __restrict__ pres, PciBuffers b, PciOut o) {
-  uint32_t p, sc;
-  bool lead;
-  if (!map.locate(n, p, sc, lead)) return;
-  map.patch(c, sc);
-  if (!REF && is_boundary(c, b.aid, p)) {
-    // rigid-sphere boundary particle: static during the corrector
-    const float4 x = xs[p];
-    b.anp[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-    b.dl[p] = 0.f;
-    b.xp0[p] = make_float4(x.x, x.y, x.z, 0.f);
-    if (FEAT)
-      for (int k = 1; k < 8; ++k) b.feat[(size_t)k * n + p] = 0.f;
-    return;
-  }
-  // the compact list unless this scene's offsets overflowed it (or, once
-  // they have, the search writes the grouped 32-bit list instead)
-  const PciStatus* stc = b.st ? b.st + map.scene_of_block() : nullptr;
-  const bool c16 = b.list16 && stc && stc->wide == 0u && !(M::kWideList && c.list32g && stc->want32);
-  const uint32_t m = cnt[p];
-  PairSums s;
-  float dl = c.delta;
-  if (REF) {
-    s = c16 ? internal_sums_l<false, SURF>(c, p, n, m, List16{b.list16, n}, xs, vs)
-            : internal_sums_l<false, SURF>(c, p, n, m, List32{list, n}, xs, vs);
-  } else {
-    s = c16 ? np_sums<SURF, FEAT>(c, p, n, m, List16{b.list16, n}, xs, vs, b.feat, dl)
-            : np_sums<SURF, FEAT>(c, p, n, m, List32{list, n}, xs, vs, b.feat, dl);
-  }
+// The end of the non-pressure pass for particle p: its force densities and
+// the first prediction.
+template <bool REF, bool SURF, bool WARM, bool OUT>
+__device__ __forceinline__ void np_finish(uint32_t p, const Consts& c, const PairSums& s, float dl,
+                                          const float4* __restrict__ xs,
+                                          const float* __restrict__ rho,
+                                          const float4* __restrict__ avh,
+                                          const float* __restrict__ pres, const PciBuffers& b,
+                                          const PciOut& o) {
   const float ri = rho[p];
   const float sigma = REF ? 0.0728f : c.sigma;
   float fV[3] = {s.fv[0] * c.cv, s.fv[1] * c.cv, s.fv[2] * c.cv};
@@ -228,6 +205,153 @@ __global__ __launch_bounds__(M::kMaxThreads) void k_pci_nonpressure(
     if (o.fV) o.fV[p] = make_float4(fV[0], fV[1], fV[2], 0.f);
     if (o.fS) o.fS[p] = make_float4(fS[0], fS[1], fS[2], 0.f);
   }
+}
+
+// A rigid-sphere boundary particle: static during the corrector.
+__device__ __forceinline__ void np_boundary(uint32_t p, const float4* __restrict__ xs,
+                                            const PciBuffers& b) {
+  const float4 x = xs[p];
+  b.anp[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+  b.dl[p] = 0.f;
+  b.xp0[p] = make_float4(x.x, x.y, x.z, 0.f);
+}
+
+// compute_Viscosity_SurfaceTension_Force_PCI (PciSphSystem_Kernel.cu:117-170)
+// + first prediction (integrateSPH_LeapFrog_Forces with f_P = 0).
+template <bool REF, bool SURF, bool WARM, bool OUT, bool FEAT, class M>
+__global__ __launch_bounds__(M::kMaxThreads) void k_pci_nonpressure(
+    M map, uint32_t n, Consts c, const uint32_t* __restrict__ cnt,
+    const uint32_t* __restrict__ list, const float4* __restrict__ xs,
+    const float4* __restrict__ vs, const float* __restrict__ rho, const float4* __restrict__ avh,
+    const float* __restrict__ pres, PciBuffers b, PciOut o) {
+  uint32_t p, sc;
+  bool lead;
+  if (!map.locate(n, p, sc, lead)) return;
+  map.patch(c, sc);
+  if (!REF && is_boundary(c, b.aid, p)) {
+    np_boundary(p, xs, b);
+    if (FEAT)
+      for (int k = 1; k < 8; ++k) b.feat[(size_t)k * n + p] = 0.f;
+    return;
+  }
+  // the compact list unless this scene's offsets overflowed it (or, once
+  // they have, the search writes the grouped 32-bit list instead)
+  const PciStatus* stc = b.st ? b.st + map.scene_of_block() : nullptr;
+  const bool c16 = b.list16 && stc && stc->wide == 0u && !(M::kWideList && c.list32g && stc->want32);
+  const uint32_t m = cnt[p];
+  PairSums s;
+  float dl = c.delta;
+  if (REF) {
+    s = c16 ? internal_sums_l<false, SURF>(c, p, n, m, List16{b.list16, n}, xs, vs)
+            : internal_sums_l<false, SURF>(c, p, n, m, List32{list, n}, xs, vs);
+  } else {
+    s = c16 ? np_sums<SURF, FEAT>(c, p, n, m, List16{b.list16, n}, xs, vs, b.feat, dl)
+            : np_sums<SURF, FEAT>(c, p, n, m, List32{list, n}, xs, vs, b.feat, dl);
+  }
+  np_finish<REF, SURF, WARM, OUT>(p, c, s, dl, xs, rho, avh, pres, b, o);
+}
+
+// The same for few particles, eight lanes to one (as the WCSPH force pass):
+// the lanes take eight list entries at a time and leave the pairs' factors in
+// LDS, then seven of them add one sum each over the eight in list order --
+// three of viscosity and, in reference mode, four of surface tension, else
+// four of the pressure scaling.  Without the warm-start features, and in
+// config mode without surface tension.
+// Bound by latency at 4,096 particles (6.6 us, one lane 13.7), by instruction
+// issue at 64,000 (12.6 against 14.9).
+constexpr int kNpLanes = 8;
+constexpr uint32_t kNpP = 256 / kNpLanes;   // particles per workgroup
+template <bool REF, bool WARM, bool OUT>
+__global__ __launch_bounds__(256) void k_pci_nonpressure_lanes(
+    uint32_t n, Consts c, const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ list,
+    const float4* __restrict__ xs, const float4* __restrict__ vs, const float* __restrict__ rho,
+    const float4* __restrict__ avh, const float* __restrict__ pres, PciBuffers b, PciOut o) {
+  constexpr uint32_t L = kNpLanes, F = REF ? 12 : 8;   // floats per pair
+  // 8 words of padding keep the particles of a wave on different banks
+  __shared__ __align__(16) float pairs[kNpP][L * F + 8];
+  const uint32_t lane = threadIdx.x % L, slot = threadIdx.x / L;
+  const uint32_t p = xcd_block(blockIdx.x, gridDim.x) * kNpP + slot;
+  const uint32_t pc = min(p, n - 1u);
+  const bool fixed = !REF && p < n && is_boundary(c, b.aid, p);
+  const uint32_t m = p < n && !fixed ? cnt[p] : 0u;
+  const bool c16 = b.list16 && b.st && b.st->wide == 0u && !(c.list32g && b.st->want32);
+  const float4 xi = xs[pc], vi = vs[pc];
+  // entry k, the last one past the end (the particle itself without entries)
+  auto entry = [&](uint32_t k) {
+    if (!m) return pc;
+    k = min(k, m - 1u);
+    return c16 ? p + (uint32_t)b.list16[l16_at(k, p, n)] - 32768u : list[(uint64_t)k * n + p];
+  };
+  uint32_t q = entry(lane);
+  float4 xj = gather4(xs, q), vj = gather4(vs, q);
+  q = entry(lane + L);
+  float* const mine = pairs[slot];
+  // factors of a pair: velocity difference, viscosity factor; then in
+  // reference mode normal direction and factor, surface factors, else gradient
+  // and its square (added as they are)
+  const bool unit = !REF && lane >= 3u;
+  const uint32_t ca = lane < 3u ? lane : REF ? (lane < 6u ? lane + 1u : 8u) : min(lane + 1u, 7u);
+  const uint32_t cb = lane < 3u ? 3u : REF ? (lane < 6u ? 7u : 9u) : 0u;
+  const bool local = c.delta_local_cap;
+  const bool bodies = c.n_fluid != kNoBodies;
+  float sum = 0.f;
+  for (uint32_t k0 = 0; __any(k0 < m); k0 += L) {
+    const float4 xn = gather4(xs, q), vn = gather4(vs, q);
+    q = entry(k0 + 2u * L + lane);
+    const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+    const float d2 = dot3(dx, dy, dz, dx, dy, dz);
+    // pairs that add nothing have all factors 0
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 f0 = zero, f1 = zero, f2 = zero;
+    if (d2 > 0.f && k0 + lane < m) {
+      float dd, invd = 0.f;
+      if (!REF && local) dist_and_inverse(d2, dd, invd);
+      else dd = sqrt_rn(d2);
+      const float hd = c.h - dd;
+      f0 = make_float4(vj.x - vi.x, vj.y - vi.y, vj.z - vi.z, hd * vj.w);
+      if (REF) {
+        const float a = c.h2 - d2;
+        f1 = make_float4(dx, dy, dz, (a * a) * vj.w);
+        f2.x = a * (c.h2x3 - 7.0f * d2);
+        f2.y = vj.w;
+      } else if (local && d2 < c.h2) {
+        const float gw = c.c_spiky * (hd * hd);
+        f1.x = (dx * invd) * gw; f1.y = (dy * invd) * gw; f1.z = (dz * invd) * gw;
+        if (!bodies || vj.w > 0.f) f1.w = dot3(f1.x, f1.y, f1.z, f1.x, f1.y, f1.z);
+      }
+    }
+    float4* const row = reinterpret_cast<float4*>(mine + F * lane);
+    row[0] = f0;
+    row[1] = f1;
+    if (REF) row[2] = f2;
+    wave_lds_order();
+#pragma unroll
+    for (uint32_t e = 0; e < L; ++e)
+      sum = __builtin_fmaf(mine[F * e + ca], unit ? 1.f : mine[F * e + cb], sum);
+    wave_lds_order();
+    xj = xn;
+    vj = vn;
+  }
+  float t[7];
+#pragma unroll
+  for (int k = 0; k < 7; ++k) t[k] = __shfl(sum, k, kNpLanes);
+  if (lane != 0u || p >= n) return;
+  if (fixed) {
+    np_boundary(p, xs, b);
+    return;
+  }
+  PairSums s;
+  s.fp[0] = s.fp[1] = s.fp[2] = 0.f;
+  s.fs = s.nn[0] = s.nn[1] = s.nn[2] = 0.f;
+  s.fv[0] = t[0]; s.fv[1] = t[1]; s.fv[2] = t[2];
+  float dl = c.delta;
+  if (REF) {
+    s.nn[0] = t[3]; s.nn[1] = t[4]; s.nn[2] = t[5];
+    s.fs = t[6];
+  } else {
+    dl = np_delta(c, xi, t[3], t[4], t[5], t[6]);
+  }
+  np_finish<REF, REF, WARM, OUT>(p, c, s, dl, xs, rho, avh, pres, b, o);
 }
 
 // compute_Density_PCI + compute_Pressure_PCI (PciSphSystem_Kernel.cu:36-85)
@@ -638,6 +762,26 @@ psb_status launch_pci_nonpressure(uint32_t n, const Consts& c, bool surf, bool w
                                   const float4* vs, const float* rho, const float4* avh,
                                   const float* pres, const PciBuffers& b, const PciOut& o,
                                   hipStream_t s) {
+  if (!n) return PSB_OK;
+  int dev = 0, cus = 0;
+  PSB_HIP(hipGetDevice(&dev));
+  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const bool ref = c.mode == PSB_MODE_REFERENCE;
+  // eight lanes per particle up to 256 particles a compute unit (one lane ->
+  // eight, us: config 4,096 13.7 -> 6.6, 32,768 14.2 -> 9.6, 64,000 14.9 ->
+  // 12.6, 110,592 16.9 -> 18.9; reference 1,000 11.4 -> 5.7, 43,993 13.0 ->
+  // 9.8, 85,184 14.5 -> 14.8)
+  if (n <= 256ull * (uint64_t)cus && (ref || (!surf && !b.feat))) {
+#define PSB_NPL(R_, W_, O_)                                                                       \
+  hipLaunchKernelGGL((k_pci_nonpressure_lanes<R_, W_, O_>), dim3(blocks_for(n, kNpP)), dim3(256), 0, \
+                     s, n, c, cnt, list, xs, vs, rho, avh, pres, b, o)
+    if (ref) { if (out) PSB_NPL(true, false, true); else PSB_NPL(true, false, false); }
+    else if (warm) { if (out) PSB_NPL(false, true, true); else PSB_NPL(false, true, false); }
+    else { if (out) PSB_NPL(false, false, true); else PSB_NPL(false, false, false); }
+#undef PSB_NPL
+    PSB_HIP(hipGetLastError());
+    return PSB_OK;
+  }
   return nonpressure_impl(SingleMap{}, single_shape(n), n, c, surf, warm, out, cnt, list, xs, vs,
                           rho, avh, pres, b, o, s);
 }

@@ -56,3 +56,20 @@ def test_wcsph_on_both_sides_of_the_rule(ctx, oracle, n):
     a, b = g.state(), o.state()
     for k in ("pos", "vel", "density", "ids"):
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("mode", [MODE_CONFIG, MODE_REFERENCE])
+@pytest.mark.parametrize("n", [65536, 65537])
+def test_pcisph_on_both_sides_of_the_rule(ctx, oracle, n, mode):
+    from psb_project_amd.system import FluidSystem
+    p = scenes.pcisph_dam_break(n_side=41, mode=mode, retry_levels=0)
+    x, p = p.pos4[:n].copy(), p.params
+    p.max_iterations = 3
+    x[:, :3] += np.random.default_rng(n).uniform(-3e-4, 3e-4, (n, 3)).astype(np.float32)
+    g, o = FluidSystem(ctx, p, n), oracle.OracleSystem(p, n)
+    for s in (g, o):
+        s.set_particles(x)
+        s.update(1)
+    a, b = g.state(), o.state()
+    for k in ("pos", "vel", "density", "pressure", "ids"):
+        assert np.array_equal(a[k], b[k]), k
