@@ -918,10 +918,11 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   //                      -> 27.3  157,464 39.0 -> 37.4  195,112 40.8 -> 44.5
   // (cells of the radius: 32,768 31.9 -> 10.9 and 34.3 -> 13.4, 110,592 39.2
   // -> 23.6 and 40.9 -> 31.8, 262,144 58.7 -> 45.4 and 59.0 -> 66.0).  Staged
-  // tiles keep the plain search.
+  // tiles, and more particles than gather4 reaches, keep the plain search.
   int cus = 0;
   PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->ctx->device));
-  if (!tiles && (R == 1 || R == 2) && (!rho || n <= 576ull * (uint64_t)cus)) {
+  if (!tiles && (R == 1 || R == 2) && n <= kMaxParticles &&
+      (!rho || n <= 576ull * (uint64_t)cus)) {
 #define PSB_NBS(D_, R_)                                                                           \
   hipLaunchKernelGGL((k_neighbors_split<D_, R_>), dim3(blocks_for(n, 64u)),                       \
                      dim3(64 * kSplit), 0, s, xs, n, gd, g->start, r2, nb.capacity, \

@@ -925,13 +925,13 @@ __device__ __forceinline__ void for_neighbors_split(uint32_t p, uint32_t n, uint
     walk_list<V>(p, n, m, list.l, [&](const uint32_t (&q)[V]) {
       float4 xq[V];
 #pragma unroll
-      for (int u = 0; u < V; ++u) xq[u] = gather4(X, q[u]);
+      for (int u = 0; u < V; ++u) xq[u] = X[q[u]];
 #pragma unroll
       for (int u = 0; u < V; ++u) f(u & 1, xq[u]);
     }, [&](const uint32_t (&q)[V], uint32_t r) {
       float4 xq[V];
 #pragma unroll
-      for (int u = 0; u < V; ++u) xq[u] = gather4(X, q[u]);
+      for (int u = 0; u < V; ++u) xq[u] = X[q[u]];
 #pragma unroll
       for (int u = 0; u < V; ++u)
         if ((uint32_t)u < r) f(u & 1, xq[u]);
@@ -1003,13 +1003,13 @@ __device__ __forceinline__ void for_pairs2(uint32_t p, uint32_t n, uint32_t m, c
     walk_list<U>(p, n, m, list.l, [&](const uint32_t (&q)[U]) {
       float4 xq[U], vq[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) { xq[u] = gather4(X, q[u]); vq[u] = gather4(V, q[u]); }
+      for (int u = 0; u < U; ++u) { xq[u] = X[q[u]]; vq[u] = V[q[u]]; }
 #pragma unroll
       for (int u = 0; u < U; ++u) f(xq[u], vq[u]);
     }, [&](const uint32_t (&q)[U], uint32_t r) {
       float4 xq[U], vq[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) { xq[u] = gather4(X, q[u]); vq[u] = gather4(V, q[u]); }
+      for (int u = 0; u < U; ++u) { xq[u] = X[q[u]]; vq[u] = V[q[u]]; }
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if ((uint32_t)u < r) f(xq[u], vq[u]);

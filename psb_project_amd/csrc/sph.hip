@@ -47,13 +47,13 @@ __global__ __launch_bounds__(256) void k_density_list(uint32_t n, Consts c,
   walk_list<kWide>(p, n, m, list, [&](const uint32_t (&q)[kWide]) {
     float4 xq[kWide];
 #pragma unroll
-    for (int u = 0; u < kWide; ++u) xq[u] = gather4(pos, q[u]);
+    for (int u = 0; u < kWide; ++u) xq[u] = pos[q[u]];
 #pragma unroll
     for (int u = 0; u < kWide; ++u) add(xq[u]);
   }, [&](const uint32_t (&q)[kWide], uint32_t r) {
     float4 xq[kWide];
 #pragma unroll
-    for (int u = 0; u < kWide; ++u) xq[u] = gather4(pos, q[u]);
+    for (int u = 0; u < kWide; ++u) xq[u] = pos[q[u]];
 #pragma unroll
     for (int u = 0; u < kWide; ++u)
       if ((uint32_t)u < r) add(xq[u]);
