@@ -102,7 +102,18 @@ struct NodeGrid {
   int nx, ny, nz;
   float ox, oy, oz, cell;
   float iso, r2, inv_r6;
+  float edge2;   // near_edge of r2
 };
+
+// The d^2 above which a particle closer than r may lie outside a point's 27
+// cells.  An index (x - min) / r carries two roundings, so it is off by at most
+// 2^-23 of itself: of two points in a grid of `cells` along its longest axis
+// the one more than a cell away is no nearer than (1 - 2^-22 cells) r.  Above
+// 2,000 cells that is less than 0.999 of r^2, which 16,000 cells do pass.
+inline float near_edge(float r2, int cells) {
+  const double share = 1.0 - (double)cells / (1 << 21) - 1.0 / (1 << 18);
+  return r2 * (float)std::max(0.0, std::min(0.999, share));
+}
 
 __device__ __forceinline__ void node_pos(const NodeGrid& G, int i, int j, int k, float& x, float& y,
                                          float& z) {
@@ -192,8 +203,7 @@ __device__ __forceinline__ void for_near_box(const GridDev& g, const uint32_t* _
 
 // Whether particle x lies in the 27 cells around the point whose cell is c.  A
 // particle outside them is more than a cell (r) away but for rounding at the
-// cell borders: only a distance this close to r needs the test.
-constexpr float kNearEdge = 0.999f;
+// cell borders: only a d^2 above NodeGrid::edge2 needs the test (near_edge).
 __device__ __forceinline__ bool in_cells(const GridDev& g, const int (&c)[3], const float4& x) {
   uint32_t bad = 0;
   const int kx = cell_coord(x.x, g.minx, g.cell, g.nx, bad);
@@ -240,7 +250,7 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_iso(NodeGrid G, GridDev g,
   int c[3];
   cells_of(g, x, y, z, c);
   float acc = 0.f;
-  const float edge2 = G.r2 * kNearEdge;
+  const float edge2 = G.edge2;
   for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
     const float dx = x - q.x, dy = y - q.y, dz = z - q.z;
     const float d2 = dot3(dx, dy, dz, dx, dy, dz);
@@ -301,7 +311,7 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_vertices(
   node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
   node_pos(G, o[0] + kNodeBlock, o[1] + kNodeBlock, o[2] + kNodeBlock, w.hi[0], w.hi[1], w.hi[2]);
   box_cells(g, w);
-  const float edge2 = G.r2 * kNearEdge;
+  const float edge2 = G.edge2;
   for (uint32_t v0 = 0; v0 < total; v0 += 64u) {
     const bool on = v0 + lane < total;
     const uint32_t ed = edge[wv][on ? v0 + lane : v0];
@@ -569,6 +579,7 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   gd.cell_size = r;
   PSB_ARG((uint64_t)gd.dims[0] * gd.dims[1] * gd.dims[2] <= (1ull << 31),
           "particle grid too fine for the surface radius");
+  G.edge2 = near_edge(G.r2, std::max(gd.dims[0], std::max(gd.dims[1], gd.dims[2])));
   if (!s->grid || std::memcmp(&gd, &s->gdesc, sizeof gd) != 0 || n > s->grid_cap) {
     if (s->grid) { psb_finalize_grid(s->grid); s->grid = nullptr; }
     PSB_TRY(psb_create_grid_desc(s->ctx, &gd, n, &s->grid));

@@ -33,3 +33,58 @@ def test_node_blocks_bitwise(ctx, oracle, n, side, cell, left_out):
     else:
         same(s.extract_points(x, 0.02, p), oracle.surface_extract(x, 0.02, p))
     s.close()
+
+
+def border_pairs(ratio, n_nodes, x0, h):
+    """A row of particles along x whose grid has ratio * n_nodes cells: two
+    ends, and beside some nodes a particle closer than r (d^2 < 0.9988 r^2) that
+    the rounded cell indexes put two cells away from the node."""
+    f = np.float32
+    p = surface.default_params(cell_size=0.0)
+    p.scale = 1.0
+    r = f(h) / f(p.scale)
+    p.cell_size = float(r) * ratio
+    cell = f(p.cell_size)
+    p.margin = (1.4999 * p.cell_size - 0.01) / float(r)   # three nodes across, one in the middle
+    mid = 1.4
+    lo = np.array([x0, mid, mid], np.float32)
+    hi = np.array([lo[0] + n_nodes * p.cell_size, mid + 0.02, mid + 0.02], np.float32)
+    margin = float(f(p.margin)) * float(r)
+    mn = [float(lo[a]) - margin for a in range(3)]
+    mx = [float(hi[a]) + margin for a in range(3)]
+    org = [f((mn[a] + mx[a]) / 2 - abs(mx[a] - mn[a]) / 2 + float(cell) / 2) for a in range(3)]
+    nodes = [org[a] + np.arange(int(np.ceil((mx[a] - mn[a]) / float(cell))), dtype=f) * cell
+             for a in range(3)]
+    # the node row within the particles' y, z range
+    y, z = (nodes[a][np.argmin(np.abs(nodes[a] - mid - 0.01))] for a in (1, 2))
+    assert lo[1] <= y <= hi[1] and lo[2] <= z <= hi[2]
+
+    def index(x):
+        return np.floor((x - f(mn[0])) / r)
+
+    x = nodes[0][(nodes[0] > lo[0]) & (nodes[0] < hi[0] - 1)]
+    q = (float(f(mn[0])) + (index(x) + 2).astype(np.float64) * float(r)).astype(f)   # that border
+    found = []
+    for step in (-np.inf, np.inf):
+        c = q
+        for _ in range(4):
+            d = x - c
+            found.append(c[(d * d < f(0.9988) * r * r) & (index(c) - index(x) >= 2)])
+            c = np.nextafter(c, f(step))
+    found = np.unique(np.concatenate(found))
+    pts = np.zeros((2 + found.size, 4), f)
+    pts[0, :3], pts[1, :3] = lo, hi
+    pts[2:, 0], pts[2:, 1], pts[2:, 2] = found, y, z
+    return pts, h, p, found.size
+
+
+@pytest.mark.parametrize("ratio,x0,h", [(14.173, 2.794, 0.01216), (10.0, -1.815, 0.01293),
+                                        (4.08, 2.384, 0.02249)])
+def test_cell_borders_of_wide_grids(ctx, oracle, ratio, x0, h):
+    """Particles within r of a node, outside its 27 cells by the rounding of
+    the cell index (16,000 to 57,000 cells on an axis), add nothing."""
+    x, h, p, pairs = border_pairs(ratio, 4000, x0, h)
+    assert pairs > 0
+    s = surface.Surface(ctx)
+    same(s.extract_points(x, h, p), oracle.surface_extract(x, h, p))
+    s.close()
