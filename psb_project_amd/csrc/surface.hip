@@ -9,12 +9,13 @@
 //   k_sorted     particles in the order of a uniform grid of cell r
 //   k_iso        field at each node, f = sum_j (r^2 - d_j^2)^3 / r^6 over
 //                the particles within r = h / scale (27 cells), in sorted
-//                order; one wave per 4 x 4 x 4 nodes
+//                order; one wave per 4 x 4 x 4 nodes, which takes its
+//                candidates together where nodes are close (kBoxCells)
 //   k_edges      crossed grid edges (one end <= iso, the other not), three
 //                per node (+x, +y, +z); exclusive scan -> vertex numbers
 //   k_vertices   one vertex per crossed edge, vertexInterpolate_MarchingCube
 //                (MarchingCube_Kernel.cu:145-155), and its normal: the
-//                direction of -grad f; one wave per 4 x 4 x 4 nodes
+//                direction of -grad f; waves and candidates as for k_iso
 //   k_cubes      case index and triangle count per cube; exclusive scan
 //   k_emit       triangles as vertex-index triples, cube by cube (x fastest)
 //
@@ -159,7 +160,7 @@ __device__ __forceinline__ void box_cells(const GridDev& g, WaveBox& w) {
 // of the box go to LDS in order, and every lane then sees each of them (an
 // LDS broadcast).  The field and normal sums of a lane's own 27 cells are
 // ~780 candidates at r = 3 spacings of which ~120 lie within r; per wave ~620
-// are near a block of 4^3 nodes, and one load serves 64 nodes instead of a
+// are near a block of 4^3 nodes a third of r apart, and one load serves 64 nodes instead of a
 // gather (through the permutation) per candidate and node.  262,144 particles,
 // 440,000 nodes: k_iso 617 -> 106 us, k_vertices 245 -> 57 us; what is left
 // is the ~13 VALU instructions per wave and survivor.
@@ -218,6 +219,28 @@ __device__ __forceinline__ void cells_of(const GridDev& g, float x, float y, flo
   c[2] = cell_coord(z, g.minz, g.cell, g.nz, bad);
 }
 
+// The same for each lane by itself: the particles of the 27 cells around c in
+// sorted order, four loads in flight (at one spacing per cell bound by their
+// latency).
+template <class F>
+__device__ __forceinline__ void for_near_cells(const GridDev& g, const uint32_t* __restrict__ start,
+                                               const float4* __restrict__ xs, const int (&c)[3],
+                                               F&& f) {
+  const int x0 = max(c[0] - 1, 0), x1 = min(c[0] + 1, g.nx - 1);
+  for (int zz = max(c[2] - 1, 0); zz <= min(c[2] + 1, g.nz - 1); ++zz)
+    for (int yy = max(c[1] - 1, 0); yy <= min(c[1] + 1, g.ny - 1); ++yy) {
+      const uint64_t base = (uint64_t)g.nx * ((uint64_t)yy + (uint64_t)g.ny * (uint64_t)zz);
+      const uint32_t q1 = start[base + x1 + 1];
+      for (uint32_t q = start[base + x0]; q < q1; q += 4u) {
+        float4 x[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) x[u] = xs[min(q + u, q1 - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) f(x[u], q + u < q1);
+      }
+    }
+}
+
 // first node of wave `w`'s block (blocks x fastest), false past the last block
 __device__ __forceinline__ bool block_origin(const NodeGrid& G, uint32_t w, int (&o)[3]) {
   const uint32_t bx = (G.nx + kNodeBlock - 1) / kNodeBlock, by = (G.ny + kNodeBlock - 1) / kNodeBlock,
@@ -229,27 +252,46 @@ __device__ __forceinline__ bool block_origin(const NodeGrid& G, uint32_t w, int 
 }
 
 constexpr uint32_t kIsoWaves = 4;   // waves per workgroup, one node block each
+template <bool BOX>
 __global__ __launch_bounds__(64 * kIsoWaves) void k_iso(NodeGrid G, GridDev g,
                                                         const uint32_t* __restrict__ start,
                                                         const float4* __restrict__ xs,
                                                         float* __restrict__ iso) {
-  __shared__ float4 lds[kIsoWaves][64 + 4];
+  __shared__ float4 lds[BOX ? kIsoWaves : 1][BOX ? 64 + 4 : 1];
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int o[3];
   if (!block_origin(G, blockIdx.x * kIsoWaves + wv, o)) return;
+  const int i = o[0] + (int)(lane & 3u), j = o[1] + (int)(lane >> 2 & 3u), k = o[2] + (int)(lane >> 4);
+  const bool mine = i < G.nx && j < G.ny && k < G.nz;
+  float x, y, z;
+  node_pos(G, i, j, k, x, y, z);
+  int c[3];
+  cells_of(g, x, y, z, c);
+  float acc = 0.f;
+  if constexpr (!BOX) {
+    if (!mine) return;
+    // (the weight in a function of its own: written into the walk it came out
+    // with a branch per candidate, 284 against 252 us an extraction at a
+    // spacing of r)
+    auto add = [&](float d2, bool in) {
+      const float v = in ? G.r2 - d2 : 0.f;
+      acc = __builtin_fmaf(v * v, v, acc);   // v = 0 leaves acc (never -0) unchanged
+    };
+    for_near_cells(g, start, xs, c, [&](const float4& q, bool in) {
+      const float dx = x - q.x, dy = y - q.y, dz = z - q.z;
+      const float d2 = dot3(dx, dy, dz, dx, dy, dz);
+      add(d2, in && d2 <= G.r2);
+    });
+    iso[(uint64_t)i + (uint64_t)G.nx * ((uint64_t)j + (uint64_t)G.ny * (uint64_t)k)] = acc * G.inv_r6;
+    return;
+  }
   const int e[3] = {min(o[0] + kNodeBlock, G.nx) - 1, min(o[1] + kNodeBlock, G.ny) - 1,
                     min(o[2] + kNodeBlock, G.nz) - 1};
   WaveBox w;
   node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
   node_pos(G, e[0], e[1], e[2], w.hi[0], w.hi[1], w.hi[2]);
   box_cells(g, w);
-  const int i = o[0] + (int)(lane & 3u), j = o[1] + (int)(lane >> 2 & 3u), k = o[2] + (int)(lane >> 4);
-  float x, y, z;
-  node_pos(G, i, j, k, x, y, z);
-  int c[3];
-  cells_of(g, x, y, z, c);
-  float acc = 0.f;
   const float edge2 = G.edge2;
   for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
     const float dx = x - q.x, dy = y - q.y, dz = z - q.z;
@@ -257,11 +299,22 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_iso(NodeGrid G, GridDev g,
     bool in = d2 <= G.r2;
     if (__any(in && d2 > edge2)) in = in && (d2 <= edge2 || in_cells(g, c, q));
     const float v = in ? G.r2 - d2 : 0.f;
-    acc = __builtin_fmaf(v * v, v, acc);   // v = 0 leaves acc (never -0) unchanged
+    acc = __builtin_fmaf(v * v, v, acc);
   });
-  if (i < G.nx && j < G.ny && k < G.nz)
+  if (mine)
     iso[(uint64_t)i + (uint64_t)G.nx * ((uint64_t)j + (uint64_t)G.ny * (uint64_t)k)] = acc * G.inv_r6;
 }
+
+// A wave takes its block's candidates together up to this node spacing over
+// r; above, each lane walks its own 27 cells.  The box a wave has to look
+// through grows with the cube of (3 spacings + 2 r), a lane's cells do not.
+// Us per extraction, box / cells (particles; r in particle spacings):
+//                    0.25         0.4        0.5        1          4
+//   262,144; 3.1   336 / 443   275 / 298  308 / 246  850 / 253  10,450 / 219
+//   32,768; 3.1    200 / 208   264 / 218  275 / 208  777 / 230   5,860 / 214
+//   262,144; 2     340 / 423   220 / 274  208 / 195  321 / 156   2,400 / 141
+//   32,768; 5                  607 / 522  780 / 500  2,265 / 520
+constexpr float kBoxCells = 0.4f;
 
 __global__ __launch_bounds__(256) void k_edges(NodeGrid G, const float* __restrict__ iso,
                                                uint8_t* __restrict__ eflags,
@@ -281,11 +334,12 @@ __global__ __launch_bounds__(256) void k_edges(NodeGrid G, const float* __restri
 
 // One wave per node block: the block's crossed edges are dealt to the lanes
 // (a wave of consecutive nodes had ~1 lane in 10 at work), 64 at a time.
+template <bool BOX>
 __global__ __launch_bounds__(64 * kIsoWaves) void k_vertices(
     NodeGrid G, GridDev g, const uint32_t* __restrict__ start, const float4* __restrict__ xs,
     const float* __restrict__ iso, const uint8_t* __restrict__ eflags,
     const uint32_t* __restrict__ vbase, float* __restrict__ verts, float* __restrict__ norms) {
-  __shared__ float4 lds[kIsoWaves][64 + 4];
+  __shared__ float4 lds[BOX ? kIsoWaves : 1][BOX ? 64 + 4 : 1];
   __shared__ uint8_t edge[kIsoWaves][192];   // node of the block (6 bits), axis (2 bits)
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -308,9 +362,11 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_vertices(
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   WaveBox w;
-  node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
-  node_pos(G, o[0] + kNodeBlock, o[1] + kNodeBlock, o[2] + kNodeBlock, w.hi[0], w.hi[1], w.hi[2]);
-  box_cells(g, w);
+  if constexpr (BOX) {
+    node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
+    node_pos(G, o[0] + kNodeBlock, o[1] + kNodeBlock, o[2] + kNodeBlock, w.hi[0], w.hi[1], w.hi[2]);
+    box_cells(g, w);
+  }
   const float edge2 = G.edge2;
   for (uint32_t v0 = 0; v0 < total; v0 += 64u) {
     const bool on = v0 + lane < total;
@@ -336,17 +392,29 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_vertices(
     int c[3];
     cells_of(g, px, py, pz, c);
     float gx = 0.f, gy = 0.f, gz = 0.f;
-    for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
-      const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
-      const float d2 = dot3(dx, dy, dz, dx, dy, dz);
-      bool in = d2 < G.r2;
-      if (__any(in && d2 > edge2)) in = in && (d2 <= edge2 || in_cells(g, c, q));
-      const float u = in ? G.r2 - d2 : 0.f;
-      const float u2 = u * u;   // 0: adds a zero of either sign to sums that are never -0
-      gx = __builtin_fmaf(dx, u2, gx);
-      gy = __builtin_fmaf(dy, u2, gy);
-      gz = __builtin_fmaf(dz, u2, gz);
-    });
+    if constexpr (BOX) {
+      for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
+        const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+        const float d2 = dot3(dx, dy, dz, dx, dy, dz);
+        bool in = d2 < G.r2;
+        if (__any(in && d2 > edge2)) in = in && (d2 <= edge2 || in_cells(g, c, q));
+        const float u = in ? G.r2 - d2 : 0.f;
+        const float u2 = u * u;   // 0: adds a zero of either sign to sums that are never -0
+        gx = __builtin_fmaf(dx, u2, gx);
+        gy = __builtin_fmaf(dy, u2, gy);
+        gz = __builtin_fmaf(dz, u2, gz);
+      });
+    } else if (on) {
+      for_near_cells(g, start, xs, c, [&](const float4& q, bool in) {
+        const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+        const float d2 = dot3(dx, dy, dz, dx, dy, dz);
+        const float u = in && d2 < G.r2 ? G.r2 - d2 : 0.f;
+        const float u2 = u * u;
+        gx = __builtin_fmaf(dx, u2, gx);
+        gy = __builtin_fmaf(dy, u2, gy);
+        gz = __builtin_fmaf(dz, u2, gz);
+      });
+    }
     if (!on) continue;
     const float gl = sqrtf(dot3(gx, gy, gz, gx, gy, gz));
     if (gl > 0.f) { gx = gx / gl; gy = gy / gl; gz = gz / gl; }
@@ -603,8 +671,13 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   nbb = blocks_for(nbb, kIsoWaves);
   hipLaunchKernelGGL(k_sorted, dim3(blocks_for(n)), dim3(kBlock), 0, st, n, s->grid->perm, P, ids,
                      id_limit, s->xs);
-  hipLaunchKernelGGL(k_iso, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g, s->grid->start, s->xs,
-                     s->iso);
+  const bool box = prm->cell_size < kBoxCells * r;
+  if (box)
+    hipLaunchKernelGGL(k_iso<true>, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g, s->grid->start,
+                       s->xs, s->iso);
+  else
+    hipLaunchKernelGGL(k_iso<false>, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g, s->grid->start,
+                       s->xs, s->iso);
   hipLaunchKernelGGL(k_edges, dim3(nbn), dim3(kBlock), 0, st, G, s->iso, s->eflags, s->vcount);
   PSB_HIP(hipGetLastError());
   PSB_TRY(scan_exclusive(s->vcount, s->nodes, s->bsum, s->vbase, st));
@@ -621,8 +694,12 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   PSB_TRY(grow(s->verts, s->cap_v, 3 * (size_t)s->nv));
   PSB_TRY(grow(s->norms, s->cap_n, 3 * (size_t)s->nv));
   PSB_TRY(grow(s->tris, s->cap_t, 3 * (size_t)s->nt));
-  hipLaunchKernelGGL(k_vertices, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g, s->grid->start,
-                     s->xs, s->iso, s->eflags, s->vbase, s->verts, s->norms);
+  if (box)
+    hipLaunchKernelGGL(k_vertices<true>, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g,
+                       s->grid->start, s->xs, s->iso, s->eflags, s->vbase, s->verts, s->norms);
+  else
+    hipLaunchKernelGGL(k_vertices<false>, dim3(nbb), dim3(64 * kIsoWaves), 0, st, G, g,
+                       s->grid->start, s->xs, s->iso, s->eflags, s->vbase, s->verts, s->norms);
   if (s->cubes)
     hipLaunchKernelGGL(k_emit, dim3(nbc), dim3(kBlock), 0, st, G, s->iso, s->eflags, s->vbase,
                        s->tbase, s->tris);

@@ -2,10 +2,14 @@
 chunks: node grids of every remainder modulo 4, from a few nodes up, single
 particles, rows of more than 64 candidates, particles left out; bitwise
 against the oracle."""
+import ctypes as C
+import time
+
 import numpy as np
 import pytest
 
-from psb_project_amd import surface
+from psb_project_amd import scenes, surface
+from psb_project_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +92,47 @@ def test_cell_borders_of_wide_grids(ctx, oracle, ratio, x0, h):
     s = surface.Surface(ctx)
     same(s.extract_points(x, h, p), oracle.surface_extract(x, h, p))
     s.close()
+
+
+def block(n_side, spacing):
+    return scenes.lattice(n_side, spacing, origin=(0.1, 0.1, 0.1), jitter=0.1, seed=5)
+
+
+@pytest.mark.parametrize("left_out", [False, True])
+@pytest.mark.parametrize("ratio", [0.39, 0.41, 1.0, 2.5])
+def test_node_spacings_bitwise(ctx, oracle, ratio, left_out):
+    """Node spacings on both sides of the one from which every lane walks its
+    own cells, and wider than the radius."""
+    x = block((19, 14, 11), 0.01)
+    p = surface.default_params(cell_size=ratio * 0.02 / 0.65, iso_level=0.4)
+    ids = limit = None
+    if left_out:
+        ids, limit = np.random.default_rng(8).permutation(len(x)).astype(np.uint32), len(x) // 2
+    s = surface.Surface(ctx)
+    kw = {} if ids is None else dict(ids=ids, id_limit=limit)
+    ko = {} if ids is None else dict(ids=ids, limit=limit)
+    g = s.extract_points(x, 0.02, p, **kw)
+    same(g, oracle.surface_extract(x, 0.02, p, **ko))
+    assert g["triangles"].shape[0] > 10
+    s.close()
+
+
+def test_wide_node_spacing_costs_no_more(ctx):
+    """A node grid wider than the radius has a thousandth of the nodes of one
+    at a quarter of it: its extraction takes no longer (it took 29 times as
+    long while a wave looked through all of its block's box)."""
+    x = block(32, 0.01)
+    d, took = ctx.to_device(x), {}
+    for ratio in (0.25, 4.0):
+        p = surface.default_params(cell_size=ratio * 0.02 / 0.65)
+        s = surface.Surface(ctx)
+        nv, nt = C.c_uint32(), C.c_uint32()
+        best = []
+        for _ in range(8):
+            t = time.perf_counter()
+            check(lib().psb_surface_extract_points(s.handle, d.ptr, None, len(x), 0xFFFFFFFF, 0.02,
+                                                   C.byref(p), C.byref(nv), C.byref(nt)))
+            best.append(time.perf_counter() - t)
+        took[ratio] = min(best)
+        s.close()
+    assert took[4.0] < 4 * took[0.25], took
