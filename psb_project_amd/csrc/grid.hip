@@ -307,6 +307,11 @@ __global__ __launch_bounds__(256) void k_rank_reorder(const uint32_t* __restrict
   }
 }
 
+// (in a wide scene every wave comes here: most find the word set)
+__device__ __forceinline__ void report_wide(uint32_t* word) {
+  if (!__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(word, 1u);
+}
+
 // End of a particle's search: count, density (with the epilogue fused), flags.
 // (x.w written by the epilogue is not read by the search: it tests positions
 // only.)
@@ -328,7 +333,7 @@ __device__ __forceinline__ void search_finish(const M& map, uint32_t p, uint32_t
     }
   }
   if (cnt > cap) atomicOr(flags, PSB_FLAG_NEIGHBOR_OVERFLOW);
-  if (wide) atomicOr(c16.wide + (size_t)sc * c16.wide_stride, 1u);
+  if (wide) report_wide(c16.wide + (size_t)sc * c16.wide_stride);
 }
 
 // Workgroup maximum of the neighbour counts, then one atomic per workgroup on
@@ -476,20 +481,27 @@ __global__ __launch_bounds__(M::kMaxThreads) void k_neighbors(M map, const float
 // run side by side, and what is left in sequence is the density sum over its
 // neighbours' weights.
 //
-// Every lane keeps its accepted candidates (index less the particle's) in
-// LDS.  The counts of a particle's lanes, in row order, place them in the
-// list; the waves take eight of a particle's entries each, write them (whole
-// words of the compact list, rows of 64 in the plain one) and leave their
-// weights in LDS, which the first wave adds in list order: list and sum are
-// the plain search's.  40 KB a workgroup, so that four fit a compute unit.
-// Where a buffer does not hold all (more accepted candidates, or an index too
-// far away), the particle's lanes write their own entries, and the lane of
-// that buffer walks its rows again.
+// Every lane keeps its accepted candidates in LDS, as 16-bit distances from the
+// first candidate of its run of rows.  The rows of a run lie in one layer of
+// cells, so the distance spans a few rows of particles and not the layers
+// between (180 x 100 x 4 particles, whose layers are 18,000 apart: with the
+// distance from the particle itself no buffer held its candidates, and the
+// search with the density sum took 57 us against 29 for a lane per particle;
+// now 22).  The counts of a particle's runs, in row order, place the entries in
+// the list.  The waves take eight of a particle's entries each, write them
+// (whole words of the compact list, rows of 64 in the plain one) and leave their
+// weights in LDS, which the first wave adds in list order, 40 at a time: list
+// and sum are the plain search's.  40 KB a workgroup, so that four fit a compute
+// unit.
+// Where a lane accepts more than its buffer holds, the particle's lanes write
+// their own entries, that lane walking its rows again, and the weights are
+// taken from the list written (32,768 particles with 185 neighbours 161 us when
+// the first wave walked all rows by itself, now 69; a lane per particle 122).
 // Bound by latency at 1,000 particles (with the density sum 9.0 us, a lane
 // per particle 30), by instruction issue at 100,000 (27 us against 35).
 constexpr int kSplit = 5;             // lanes per particle
 constexpr uint32_t kSplitHits = 44;   // accepted candidates kept per lane
-constexpr uint32_t kSplitSum = 40;    // weights kept per particle (a multiple of 8)
+constexpr uint32_t kSplitSum = 8 * kSplit;   // weights kept per particle
 // Candidate loads in flight per stencil row (an earlier form: 6 13.7 us at
 // 32,768 particles, 8 14.5, 6 without those past the row's end 14.3).
 constexpr int kSplitSlots = 6;
@@ -497,6 +509,12 @@ template <int RT> struct SplitShape {
   static constexpr int kWidth = 2 * RT + 1;
   static constexpr int kRows = kWidth * kWidth;
   static constexpr int kPer = (kRows + kSplit - 1) / kSplit;   // rows per lane
+  // Runs of rows in one layer: one per lane, but that at RT = 1 the second
+  // lane's two rows end a layer and begin the next.
+  static constexpr bool kTwo = RT == 1;
+  static constexpr uint32_t kRuns = kTwo ? kSplit + 1 : kSplit;
+  static constexpr uint32_t lane_of(uint32_t run) { return kTwo && run >= 2u ? run - 1u : run; }
+  static __device__ uint32_t run_of(uint32_t lane) { return kTwo && lane >= 2u ? lane + 1u : lane; }
 };
 
 template <bool DENS, int RT>
@@ -507,16 +525,23 @@ __global__ __launch_bounds__(64 * kSplit) void k_neighbors_split(
     Compact16 c16, ErrSlots es, EpiArgs ep) {
   using Sh = SplitShape<RT>;
   constexpr int W = Sh::kWidth, kPer = Sh::kPer;
-  constexpr uint32_t kOver = 0x80000000u;   // flag in count: the lane's buffer does not hold all
+  constexpr uint32_t kRuns = Sh::kRuns;
   constexpr uint32_t kPitch = kSplitHits + 1;   // one more takes what does not fit
-  __shared__ int16_t rel[kSplit * kPitch * 64];
+  __shared__ uint16_t rel[kSplit * kPitch * 64];
   __shared__ float weight[DENS ? kSplitSum * 64 : 1];
-  __shared__ uint32_t count[kSplit][64];
+  // of a run: accepted candidates (6 bits) and first candidate; kOver candidates
+  // where the lane's buffer does not hold them all (it then holds their number,
+  // as 16-bit halves)
+  __shared__ uint32_t info[kRuns][64];
+  constexpr uint32_t kOver = 63u;
+  static_assert(kSplitHits < kOver && kSplitHits >= 4u && (kSplit - 1) * kPitch < 256u, "packing");
   const uint32_t i = threadIdx.x & 63u;
   const uint32_t slice = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const bool two = Sh::kTwo && slice == 1u;   // this lane's last row is a run of its own
   const uint32_t p = xcd_block(blockIdx.x, gridDim.x) * 64u + i;
   const bool valid = p < n;
-  uint32_t q0[kPer] = {}, q1[kPer] = {}, c = 0, cnt = 0;
+  uint32_t q0[kPer] = {}, q1[kPer] = {}, c = 0, c0 = 0;
+  uint32_t from = 0, from2 = 0;   // first candidate of the run (of the second one)
   float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
   int cx = 0, cy = 0, cz = 0;
   bool over = false;
@@ -534,6 +559,13 @@ __global__ __launch_bounds__(64 * kSplit) void k_neighbors_split(
     acc = d2 <= r2;
     return r2 - d2;
   };
+  // one round of kSplitSlots candidates (loads past the row's end stay inside
+  // the array and are not accepted)
+  auto load = [&](uint32_t q, float4 (&xq)[kSplitSlots]) {
+#pragma unroll
+    for (int u = 0; u < kSplitSlots; ++u) xq[u] = gather4(xs, min(q + u, n - 1u));
+  };
+  const uint32_t mine = slice * kPitch * 64u + i;
   if (valid) {
     xi = xs[p];
     uint32_t bad = 0;
@@ -542,23 +574,18 @@ __global__ __launch_bounds__(64 * kSplit) void k_neighbors_split(
     cz = cell_coord(xi.z, g.minz, g.cell, g.nz, bad);
 #pragma unroll
     for (int r = 0; r < kPer; ++r) range((int)slice * kPer + r, q0[r], q1[r]);
-    // one round of kSplitSlots candidates (loads past the row's end stay inside
-    // the array and are not accepted)
-    auto load = [&](uint32_t q, float4 (&xq)[kSplitSlots]) {
+    from = from2 = q0[kPer - 1];
 #pragma unroll
-      for (int u = 0; u < kSplitSlots; ++u) xq[u] = gather4(xs, min(q + u, n - 1u));
-    };
+    for (int r = kPer - 2; r >= 0; --r) from = two || q0[r] < q1[r] ? q0[r] : from;
     // candidates from q on, the row's last `left`
-    const uint32_t mine = slice * kPitch * 64u + i;
-    auto test = [&](uint32_t q, uint32_t left, const float4 (&xq)[kSplitSlots]) {
-      // offsets of a round reach at most kSplitSlots past its first
-      const int d = (int)(q - p);
-      over = over || d < -kCompactReach || d > kCompactReach - kSplitSlots;
+    auto test = [&](uint32_t q, uint32_t left, uint32_t first, const float4 (&xq)[kSplitSlots]) {
+      const uint32_t d = q - first;
+      over = over || d > 0xFFFFu - kSplitSlots;
 #pragma unroll
       for (int u = 0; u < kSplitSlots; ++u) {
         bool acc;
         weight_of(xq[u], acc);
-        rel[mine + 64u * min(c, kSplitHits)] = (int16_t)(d + u);
+        rel[mine + 64u * min(c, kSplitHits)] = (uint16_t)(d + u);
         c += acc && (uint32_t)u < left ? 1u : 0u;
       }
     };
@@ -568,133 +595,181 @@ __global__ __launch_bounds__(64 * kSplit) void k_neighbors_split(
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
       if (r + 1 < kPer) load(q0[r + 1], x0[(r + 1) & 1]);
+      if (Sh::kTwo && r == kPer - 1) c0 = c;
       if (q0[r] == q1[r]) continue;
-      test(q0[r], q1[r] - q0[r], x0[r & 1]);
+      const uint32_t first = Sh::kTwo && r == kPer - 1 && two ? from2 : from;
+      test(q0[r], q1[r] - q0[r], first, x0[r & 1]);
       for (uint32_t q = q0[r] + kSplitSlots; q < q1[r]; q += kSplitSlots) {
         float4 xq[kSplitSlots];
         load(q, xq);
-        test(q, q1[r] - q, xq);
+        test(q, q1[r] - q, first, xq);
       }
     }
     over = over || c > kSplitHits;
-    count[slice][i] = c | (over ? kOver : 0u);
+    const uint32_t run = Sh::run_of(slice), m = two ? c0 : c;
+    info[run][i] = from << 6 | (over ? kOver : m);
+    if (two) info[run + 1u][i] = from2 << 6 | (over ? kOver : c - c0);
+    if (over) {
+      rel[mine] = (uint16_t)m;
+      rel[mine + 64u] = (uint16_t)(m >> 16);
+      if (two) {
+        rel[mine + 128u] = (uint16_t)(c - c0);
+        rel[mine + 192u] = (uint16_t)((c - c0) >> 16);
+      }
+    }
   }
   __syncthreads();
   bool wide = false, listed = true;   // listed: every buffer of the particle holds all
-  uint32_t end[kSplit] = {}, at = 0, all = 0;
-  // entry k of the particle's list, less p
-  auto entry = [&](uint32_t k) {
-    uint32_t e = k;
-#pragma unroll
-    for (uint32_t s = 1; s < (uint32_t)kSplit; ++s)
-      e = k >= end[s - 1] ? s * kPitch + k - end[s - 1] : e;
-    return (int)rel[e * 64u + i];
-  };
+  // of a run: last entry + 1; first candidate (24 bits) and how much further an
+  // entry lies in rel than in the list (at most 4 kPitch)
+  uint32_t end[kRuns] = {}, where[kRuns] = {}, all = 0;
   if (valid) {
+    uint32_t longest = 0;
 #pragma unroll
-    for (uint32_t s = 0; s < (uint32_t)kSplit; ++s) {
-      const uint32_t m = count[s][i];
-      listed = listed && !(m & kOver);
-      at = s == slice ? all : at;
-      all += m & ~kOver;
+    for (uint32_t s = 0; s < kRuns; ++s) {
+      const uint32_t m = info[s][i], have = m & 63u;
+      longest = max(longest, have);
+      where[s] = (m & ~63u) << 2 |
+                 (Sh::lane_of(s) * kPitch + (Sh::kTwo && s == 2u ? end[1] - end[0] : 0u) - all);
+      all += have;
       end[s] = all;
     }
-    uint32_t* const l32g = (c16.list32g && c16.want32 && *c16.want32) ? c16.list32g : nullptr;
-    if (listed) {
-      for (uint32_t k0 = 8u * slice; k0 < (DENS ? all : min(all, cap)); k0 += 8u * kSplit) {
-        int d[8];
+    listed = longest < kOver;
+  }
+  // entry k of the particle's list
+  auto entry = [&](uint32_t k) {
+    uint32_t w = where[0];
 #pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) d[u] = entry(min(k0 + u, all - 1u));
-        if (DENS && k0 < kSplitSum) {
-          float4 xq[8];
+    for (uint32_t s = 1; s < kRuns; ++s) {
+      const uint32_t next = where[s];   // (a choice between the two array elements goes through scratch)
+      w = k >= end[s - 1] ? next : w;
+    }
+    return (w >> 8) + rel[(k + (w & 255u)) * 64u + i];
+  };
+  uint32_t* const l32g = (c16.list32g && c16.want32 && *c16.want32) ? c16.list32g : nullptr;
+  // the same for every wave of the workgroup, as all that follows from info is
+  if (__any(!listed)) {
+    if (!listed) {
+      uint32_t at = all = 0u;   // entries before this lane's, entries
 #pragma unroll
-          for (uint32_t u = 0; u < 8u; ++u) xq[u] = gather4(xs, p + (uint32_t)d[u]);
-#pragma unroll
-          for (uint32_t u = 0; u < 8u; ++u) {
-            bool acc;
-            weight[(k0 + u) * 64u + i] = weight_of(xq[u], acc);
-          }
-        }
-        if (k0 >= cap) continue;
-#pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u)
-          if (k0 + u < min(all, cap)) nlist[(uint64_t)(k0 + u) * n + p] = p + (uint32_t)d[u];
-        if (l32g) {
-          uint4* const dst = reinterpret_cast<uint4*>(l32g + l32g_at(k0, p, n));
-          dst[0] = make_uint4(p + d[0], p + d[1], p + d[2], p + d[3]);
-          dst[n] = make_uint4(p + d[4], p + d[5], p + d[6], p + d[7]);
-        } else if (c16.list16) {
-          uint32_t v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            v[u] = (uint32_t)(d[2 * u] + 32768) | (uint32_t)(d[2 * u + 1] + 32768) << 16;
-          *reinterpret_cast<uint4*>(c16.list16 + l16_at(k0, p, n)) = make_uint4(v[0], v[1], v[2], v[3]);
-        }
+      for (uint32_t s = 0; s < kRuns; ++s) {
+        const uint32_t m = info[s][i] & 63u;
+        const uint32_t b = (Sh::lane_of(s) * kPitch + (Sh::kTwo && s == 2u ? 2u : 0u)) * 64u + i;
+        at = s == Sh::run_of(slice) ? all : at;
+        all += m < kOver ? m : rel[b] | (uint32_t)rel[b + 64u] << 16;
       }
-    } else {
       auto put = [&](uint32_t k, uint32_t q) {
         if (k >= cap) return;
         nlist[(uint64_t)k * n + p] = q;
         if (l32g) l32g[l32g_at(k, p, n)] = q;
         else if (c16.list16) {
-          const int d = (int)(q - p);
-          const bool fits = d >= -kCompactReach && d <= kCompactReach;
-          if (fits) c16.list16[l16_at(k, p, n)] = (uint16_t)(d + 32768);
-          wide = wide || !fits;
+          const uint32_t e = q - p + 32768u;
+          c16.list16[l16_at(k, p, n)] = (uint16_t)e;
+          wide = wide || e - 1u >= 2u * kCompactReach + 1u;
         }
       };
       if (!over) {
-        for (uint32_t k = 0; k < c; ++k) put(at + k, p + (int)rel[(slice * kPitch + k) * 64u + i]);
+        for (uint32_t k = 0; k < c; ++k)
+          put(at + k, (two && k >= c0 ? from2 : from) + rel[mine + 64u * k]);
       } else {
 #pragma unroll
         for (int r = 0; r < kPer; ++r)
-          for (uint32_t q = q0[r]; q < q1[r]; ++q) {
-            bool acc;
-            weight_of(gather4(xs, q), acc);
-            if (acc) put(at++, q);
+          for (uint32_t q = q0[r]; q < q1[r]; q += kSplitSlots) {
+            float4 xq[kSplitSlots];
+            load(q, xq);
+#pragma unroll
+            for (int u = 0; u < kSplitSlots; ++u) {
+              bool acc;
+              weight_of(xq[u], acc);
+              if (acc && q + u < q1[r]) put(at++, q + u);
+            }
           }
       }
     }
-    if (wide && slice != 0u) atomicOr(c16.wide, 1u);
+    if (DENS) __syncthreads();   // the list just written is read below
   }
-  if (DENS) __syncthreads();
-  if (valid && slice == 0u) {
-    cnt = all;
-    float S = 0.f;
-    if (DENS && listed) {
-      for (uint32_t k = 0; k < min(all, kSplitSum); k += 8u) {
-        float w[8];
+  const uint32_t kept = min(all, cap);
+  // a list cut short holds no entry for the rest of the sum: rows again
+  const bool rows = DENS && !listed && all > cap;
+  float S = 0.f;
+  const uint32_t todo = DENS ? (rows ? 0u : all) : (listed ? kept : 0u);
+  for (uint32_t b0 = 0; DENS ? __any(b0 < todo) : b0 + 8u * slice < todo; b0 += kSplitSum) {
+    const uint32_t k0 = b0 + 8u * slice;
+    if (k0 < todo) {
+      uint32_t q[8];
+      if (!DENS || listed) {
 #pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) w[u] = weight[(k + u) * 64u + i];
+        for (uint32_t u = 0; u < 8u; ++u) q[u] = entry(min(k0 + u, all - 1u));
+      } else {
 #pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u)
-          if (k + u < all) S = __builtin_fmaf(w[u] * w[u], w[u], S);
+        for (uint32_t u = 0; u < 8u; ++u) q[u] = nlist[(uint64_t)min(k0 + u, all - 1u) * n + p];
       }
-      for (uint32_t k = kSplitSum; k < all; k += 8u) {
+      if (DENS) {
         float4 xq[8];
 #pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) xq[u] = gather4(xs, p + entry(min(k + u, all - 1u)));
+        for (uint32_t u = 0; u < 8u; ++u) xq[u] = gather4(xs, q[u]);
 #pragma unroll
         for (uint32_t u = 0; u < 8u; ++u) {
           bool acc;
-          const float w = weight_of(xq[u], acc);
-          if (k + u < all) S = __builtin_fmaf(w * w, w, S);
+          weight[(8u * slice + u) * 64u + i] = weight_of(xq[u], acc);
         }
       }
-    } else if (DENS) {
-      for (int r = 0; r < Sh::kRows; ++r) {
-        uint32_t lo, hi;
-        range(r, lo, hi);
-        for (uint32_t q = lo; q < hi; ++q) {
-          bool acc;
-          const float w = weight_of(gather4(xs, q), acc);
-          if (acc) S = __builtin_fmaf(w * w, w, S);
+      if (listed && k0 < kept) {
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u)
+          if (k0 + u < kept) nlist[(uint64_t)(k0 + u) * n + p] = q[u];
+        if (l32g) {
+          uint4* const dst = reinterpret_cast<uint4*>(l32g + l32g_at(k0, p, n));
+          dst[0] = make_uint4(q[0], q[1], q[2], q[3]);
+          dst[n] = make_uint4(q[4], q[5], q[6], q[7]);
+        } else if (c16.list16) {
+          uint32_t e[8], far = 0;
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u) {
+            e[u] = q[u] - p + 32768u;
+            far = max(far, e[u] - 1u);
+          }
+          // (past the list's end the last entry stands in; one cut off counts)
+          wide = wide || far >= 2u * kCompactReach + 1u;
+          *reinterpret_cast<uint4*>(c16.list16 + l16_at(k0, p, n)) =
+              make_uint4((e[0] & 0xFFFFu) | e[1] << 16, (e[2] & 0xFFFFu) | e[3] << 16,
+                         (e[4] & 0xFFFFu) | e[5] << 16, (e[6] & 0xFFFFu) | e[7] << 16);
         }
       }
     }
-    search_finish<DENS>(SingleMap{}, p, 0u, n, cnt, cap, wide, S, ncount, rho, mc, flags, c16, ep);
+    if (DENS) {
+      __syncthreads();
+      if (slice == 0u)
+        for (uint32_t k = b0; k < min(todo, b0 + kSplitSum); k += 8u) {
+          float w[8];
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u) w[u] = weight[(k - b0 + u) * 64u + i];
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u)
+            if (k + u < all) S = __builtin_fmaf(w[u] * w[u], w[u], S);
+        }
+      if (__any(b0 + kSplitSum < todo)) __syncthreads();
+    }
   }
-  report_max_count(SingleMap{}, cnt, maxcnt, es);
+  if (wide && slice != 0u) report_wide(c16.wide);
+  if (slice == 0u && rows)
+    for (int r = 0; r < Sh::kRows; ++r) {
+      uint32_t lo, hi;
+      range(r, lo, hi);
+      for (uint32_t q = lo; q < hi; q += kSplitSlots) {
+        float4 xq[kSplitSlots];
+        load(q, xq);
+#pragma unroll
+        for (int u = 0; u < kSplitSlots; ++u) {
+          bool acc;
+          const float w = weight_of(xq[u], acc);
+          if (acc && q + u < hi) S = __builtin_fmaf(w * w, w, S);
+        }
+      }
+    }
+  if (valid && slice == 0u)
+    search_finish<DENS>(SingleMap{}, p, 0u, n, all, cap, wide, S, ncount, rho, mc, flags, c16, ep);
+  report_max_count(SingleMap{}, slice == 0u ? all : 0u, maxcnt, es);
 }
 
 template <int W>
@@ -909,20 +984,30 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   dim3 gb(blocks_for(n)), tb(kBlock);
   EpiArgs e{};
   if (ep && rho) e = *ep;
-  // Several lanes per particle, for the stencils that have that kernel; with
-  // the density sum while one lane leaves the chip short of waves.  Us, one
-  // lane -> kSplit, jittered lattices, cells of half the radius:
-  //   without the sum    1,000 25.0 -> 6.1   32,768 24.7 -> 8.1   97,336 29.1
-  //                      -> 16.9  253,952 36.6 -> 32.9  474,552 65.0 -> 53.2
-  //   with it            4,096 30.5 -> 9.0   32,768 30.2 -> 12.4  97,336 34.6
-  //                      -> 27.3  157,464 39.0 -> 37.4  195,112 40.8 -> 44.5
-  // (cells of the radius: 32,768 31.9 -> 10.9 and 34.3 -> 13.4, 110,592 39.2
-  // -> 23.6 and 40.9 -> 31.8, 262,144 58.7 -> 45.4 and 59.0 -> 66.0).  Staged
-  // tiles, and more particles than gather4 reaches, keep the plain search.
+  // Several lanes per particle, for the stencils that have that kernel, while
+  // one leaves the chip short of waves.  Us, one lane -> kSplit, cells of half
+  // the radius (cells of the radius):
+  //   with the density sum     cube           4 layers       2 layers
+  //      4,096              27 -> 9 (34, 10)
+  //     47,000              28 -> 15 (35, 16)  25 -> 16 (27, 15)  17 -> 14 (17, 14)
+  //     64,000              29 -> 19 (37, 24)  26 -> 20 (28, 21)  19 -> 19 (19, 20)
+  //     97,000              33 -> 29 (41, 31)  27 -> 28 (32, 30)  21 -> 26 (21, 27)
+  //    125,000              33 -> 34 (42, 39)  28 -> 34 (33, 38)  22 -> 30 (23, 34)
+  //   without
+  //    148,000              35 -> 22 (46, 30)  29 -> 21 (36, 23)  24 -> 19 (25, 19)
+  //    262,144              41 -> 34 (57, 42)  36 -> 32 (46, 37)  29 -> 29 (32, 30)
+  //    512,000              72 -> 68 (99, 85)  63 -> 65 (76, 76)  48 -> 59 (47, 65)
+  // With the sum the line lies at 97,000, and at 65,536 where the lists are long
+  // enough for neighbour counts that do not fit the lanes' buffers: 145
+  // neighbours 123 -> 67 at 47,000, 148 -> 151 at 97,000; 268 (cells of half the
+  // radius; of the radius) 142 -> 63 (234, 92) at 8,000, 241 -> 231 (331, 273) at
+  // 47,000, 259 -> 323 (356, 412) at 64,000.  Without it at 262,144 (268: 477 ->
+  // 452).  Staged tiles keep the plain search, and so do particles whose index
+  // takes more than 24 bits.
   int cus = 0;
   PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->ctx->device));
-  if (!tiles && (R == 1 || R == 2) && n <= kMaxParticles &&
-      (!rho || n <= 576ull * (uint64_t)cus)) {
+  const uint64_t per_cu = !rho ? 1024u : nb.capacity <= 192u ? 384u : 256u;
+  if (!tiles && (R == 1 || R == 2) && n < 1u << 24 && n <= per_cu * (uint64_t)cus) {
 #define PSB_NBS(D_, R_)                                                                           \
   hipLaunchKernelGGL((k_neighbors_split<D_, R_>), dim3(blocks_for(n, 64u)),                       \
                      dim3(64 * kSplit), 0, s, xs, n, gd, g->start, r2, nb.capacity, \
@@ -940,7 +1025,7 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   if (rho) {
     if (R == 1) PSB_NB(true, 1); else if (R == 2) PSB_NB(true, 2); else PSB_NB(true, 0);
   } else {
-    PSB_NB(false, 0);
+    if (R == 1) PSB_NB(false, 1); else if (R == 2) PSB_NB(false, 2); else PSB_NB(false, 0);
   }
 #undef PSB_NB
   PSB_HIP(hipGetLastError());
