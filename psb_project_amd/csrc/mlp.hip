@@ -482,9 +482,7 @@ psb_status psb_mlp_create(psb_context ctx, uint64_t seed, psb_mlp* out) {
   if ((e = hipMalloc(&m->grad, 4 * kNumParams)) != hipSuccess) return fail(e);
   if ((e = hipMalloc(&m->m1, 4 * kNumParams)) != hipSuccess) return fail(e);
   if ((e = hipMalloc(&m->m2, 4 * kNumParams)) != hipSuccess) return fail(e);
-  if ((e = hipHostMalloc((void**)&m->h_loss, 64, hipHostMallocMapped | hipHostMallocCoherent)) != hipSuccess)
-    return fail(e);
-  if ((e = hipHostGetDevicePointer((void**)&m->d_loss, m->h_loss, 0)) != hipSuccess) return fail(e);
+  if ((e = take_line(ctx, (void**)&m->h_loss, (void**)&m->d_loss)) != hipSuccess) return fail(e);
   const size_t fb = sizeof(bf16x4) * 64 * 36 + 4 * kHid;
   if ((e = hipMalloc(&m->frag_mem, fb)) != hipSuccess) return fail(e);
   bf16x4* fm = (bf16x4*)m->frag_mem;
@@ -519,7 +517,7 @@ psb_status psb_mlp_destroy(psb_mlp m) {
   hipSetDevice(m->ctx->device);
   hipStreamSynchronize(m->ctx->stream);
   hipFree(m->w); hipFree(m->grad); hipFree(m->m1); hipFree(m->m2);
-  if (m->h_loss) hipHostFree(m->h_loss);
+  if (m->h_loss) give_line(m->ctx, m->h_loss);
   hipFree(m->frag_mem);
   if (m->part) hipFree(m->part);
   delete m;

@@ -51,6 +51,38 @@ psb_status launch_words_out(const uint32_t* a, uint32_t na, const uint32_t* b, u
   return PSB_OK;
 }
 
+constexpr size_t kPinnedBytes = 4096, kLineBytes = 64, kLineBase = 1024;
+constexpr int kLines = (int)((kPinnedBytes - kLineBase) / kLineBytes);
+static_assert(kLines <= 64, "one bit a line");
+
+hipError_t take_line(psb_context ctx, void** host, void** dev) {
+  {
+    std::lock_guard<std::mutex> lock(ctx->lines_mutex);
+    for (int k = 0; k < kLines; ++k)
+      if (!(ctx->lines_lent >> k & 1u)) {
+        ctx->lines_lent |= 1ull << k;
+        const size_t off = kLineBase + k * kLineBytes;
+        *host = reinterpret_cast<char*>(ctx->h_pinned) + off;
+        *dev = reinterpret_cast<char*>(ctx->d_pinned) + off;
+        return hipSuccess;
+      }
+  }
+  hipError_t e = hipHostMalloc(host, kLineBytes, hipHostMallocMapped | hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipHostGetDevicePointer(dev, *host, 0);
+  return e;
+}
+
+void give_line(psb_context ctx, void* host) {
+  const char* const base = reinterpret_cast<char*>(ctx->h_pinned) + kLineBase;
+  const size_t off = (size_t)((const char*)host - base);
+  if ((const char*)host >= base && off < kLines * kLineBytes) {
+    std::lock_guard<std::mutex> lock(ctx->lines_mutex);
+    ctx->lines_lent &= ~(1ull << off / kLineBytes);
+  } else if (host) {
+    (void)hipHostFree(host);
+  }
+}
+
 psb_status ensure_scratch(psb_context ctx, size_t bytes) {
   if (ctx->scratch_bytes >= bytes) return PSB_OK;
   if (ctx->scratch) PSB_HIP(hipFree(ctx->scratch));
@@ -323,7 +355,8 @@ psb_status psb_init(int32_t device, psb_context* out) {
   if (e != hipSuccess) { delete ctx; return hip_fail(e, "hipStreamCreate", __FILE__, __LINE__); }
   e = hipMalloc(&ctx->d_flags, 64);
   if (e == hipSuccess)
-    e = hipHostMalloc((void**)&ctx->h_pinned, 4096, hipHostMallocMapped | hipHostMallocCoherent);
+    e = hipHostMalloc((void**)&ctx->h_pinned, kPinnedBytes,
+                      hipHostMallocMapped | hipHostMallocCoherent);
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&ctx->d_pinned, ctx->h_pinned, 0);
   if (e != hipSuccess) { psb_finalize(ctx); return hip_fail(e, "context buffers", __FILE__, __LINE__); }
   // device address of this GPU's copy of the allocation-free entry point's

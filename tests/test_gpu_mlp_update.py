@@ -49,3 +49,33 @@ def test_gradient_and_adam_of_one_step(ctx, oracle, batch):
     assert np.array_equal(a, b)
     m.close()
     k.close()
+
+
+def test_many_networks_on_one_context(ctx, oracle):
+    """More networks than the context has lines for their losses (48), alive
+    together, trained in turn, some replaced: every loss is its own."""
+    rng = np.random.default_rng(4)
+    ns = 700
+    feat = rng.normal(size=(8, ns)).astype(np.float32)
+    target = rng.normal(size=ns).astype(np.float32)
+    df, dt = ctx.to_device(feat), ctx.to_device(target)
+    mean, std = np.zeros(8, np.float32), np.ones(8, np.float32)
+
+    def made(seed):
+        m = learned.PressureMLP(ctx)
+        m.set_params(he_params(seed))
+        m.set_normalization(mean, std, 1.0)
+        return m
+
+    nets = [(k, made(k)) for k in range(60)]
+    for k in (3, 50, 58):
+        nets[k][1].close()
+        nets[k] = (k + 100, made(k + 100))
+    idx = [rng.choice(ns, 64, replace=False).astype(np.uint32) for _ in nets]
+    di = [ctx.to_device(i) for i in idx]
+    losses = [m.train_step(df.ptr, dt.ptr, ns, d.ptr, 64, apply_adam=False)
+              for (_, m), d in zip(nets, di)]
+    for (seed, m), i, loss in zip(nets, idx, losses):
+        _, ref = oracle.mlp_grad(he_params(seed), mean, std, feat, target, i, emulate_bf16=True)
+        assert loss == pytest.approx(ref, rel=1e-3)
+        m.close()
