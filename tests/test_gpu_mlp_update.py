@@ -1,6 +1,8 @@
-"""The training step's update at the edges of its row groups: 1, 4, 8, 9, 64
-and 65 wave rows (batches of 16 samples a wave) and the most rows it takes,
-with and without Adam."""
+"""The training step's update at the edges of its row groups, with and without
+Adam, and many networks on one context.  The gradient pass leaves a row per
+workgroup of 64 samples (at most 512); of the update's eight threads per column
+each takes every eighth row, eight at a time: 1, 3, 8, 9, 16, 17, 57, 60, 64,
+65, 125 and 512 rows."""
 import numpy as np
 import pytest
 
@@ -10,7 +12,8 @@ from tests.test_gpu_learned import he_params
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("batch", [1, 17, 64, 144, 1024, 1030, 40000])
+@pytest.mark.parametrize("batch", [1, 17, 64, 144, 512, 513, 1024, 1030, 3648, 3840, 4096,
+                                   4097, 8000, 40000])
 def test_gradient_and_adam_of_one_step(ctx, oracle, batch):
     rng = np.random.default_rng(batch)
     ns = max(batch, 500)
