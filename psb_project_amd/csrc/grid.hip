@@ -1004,10 +1004,8 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   // 47,000, 259 -> 323 (356, 412) at 64,000.  Without it at 262,144 (268: 477 ->
   // 452).  Staged tiles keep the plain search, and so do particles whose index
   // takes more than 24 bits.
-  int cus = 0;
-  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->ctx->device));
   const uint64_t per_cu = !rho ? 1024u : nb.capacity <= 192u ? 384u : 256u;
-  if (!tiles && (R == 1 || R == 2) && n < 1u << 24 && n <= per_cu * (uint64_t)cus) {
+  if (!tiles && (R == 1 || R == 2) && n < 1u << 24 && n <= per_cu * (uint64_t)g->ctx->cus) {
 #define PSB_NBS(D_, R_)                                                                           \
   hipLaunchKernelGGL((k_neighbors_split<D_, R_>), dim3(blocks_for(n, 64u)),                       \
                      dim3(64 * kSplit), 0, s, xs, n, gd, g->start, r2, nb.capacity, \

@@ -133,7 +133,7 @@ psb_status launch_pci_nonpressure(uint32_t n, const Consts& c, bool surf, bool w
                                   const uint32_t* cnt, const uint32_t* list, const float4* xs,
                                   const float4* vs, const float* rho, const float4* avh,
                                   const float* pres, const PciBuffers& b, const PciOut& o,
-                                  hipStream_t s);
+                                  int cus, hipStream_t s);
 // density-pass flags (config mode)
 constexpr int kDensWriteFeature = 1;   // write feature 0 (first-prediction density error)
 constexpr int kDensSkipUpdate = 2;     // leave the pressure to the MLP
@@ -185,6 +185,7 @@ psb_status launch_wcsph_step_forces(uint32_t n, const Consts& c, bool surf, cons
                                     const uint32_t* list, const float4* xs, const float4* vs,
                                     const float* rho, const float* pres, const float4* avh,
                                     const uint32_t* aid, float4* bx, float4* bv, float4* bvh,
-                                    uint32_t* bid, float* bp, uint32_t* flags, hipStream_t s);
+                                    uint32_t* bid, float* bp, uint32_t* flags, int cus,
+                                    hipStream_t s);
 
 }  // namespace psb

@@ -761,11 +761,8 @@ psb_status launch_pci_nonpressure(uint32_t n, const Consts& c, bool surf, bool w
                                   const uint32_t* cnt, const uint32_t* list, const float4* xs,
                                   const float4* vs, const float* rho, const float4* avh,
                                   const float* pres, const PciBuffers& b, const PciOut& o,
-                                  hipStream_t s) {
+                                  int cus, hipStream_t s) {
   if (!n) return PSB_OK;
-  int dev = 0, cus = 0;
-  PSB_HIP(hipGetDevice(&dev));
-  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const bool ref = c.mode == PSB_MODE_REFERENCE;
   // eight lanes per particle up to 256 particles a compute unit (one lane ->
   // eight, us: config 4,096 13.7 -> 6.6, 32,768 14.2 -> 9.6, 64,000 14.9 ->
@@ -988,16 +985,14 @@ static psb_status pci_sph_update_on(psb_context ctx, const psb_sph_params* prm, 
   o.es = es;
   const bool surf = ref || prm->surface_tension != 0.f;
   PSB_TRY(launch_pci_nonpressure(n, c, surf, warm, true, nb.count, nb.list, xs, vs, density,
-                                 b.avh, pressure, b, o, s));
+                                 b.avh, pressure, b, o, ctx->cus, s));
   float4* cur = b.xp0;
   float4* nxt = xp1;
   // Two lanes per particle while one leaves the chip short of waves (reference
   // mode, density + force pass, one lane -> two: 729 particles 18.9 -> 13.9
   // us, 32,768 21.7 -> 15.7, 85,184 24.2 -> 20.3, 140,608 28.6 -> 26.9;
   // 195,112 30.6 -> 31.4, 253,952 35.1 -> 35.9)
-  int cus = 0;
-  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  const int lanes = (uint64_t)n <= 640ull * (uint64_t)cus ? 2 : 1;
+  const int lanes = (uint64_t)n <= 640ull * (uint64_t)ctx->cus ? 2 : 1;
   if (warm) {
     PSB_TRY(launch_pci_force(n, c, false, nb.count, nb.list, cur, nxt, density, pressure, b, st, -1,
                              1, o, s, lanes));

@@ -1052,6 +1052,7 @@ __device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
 
 struct psb_context_s {
   int device = 0;
+  int cus = 0;                     // its compute units
   hipStream_t stream = nullptr;
   // scratch for the standalone wrappers (grown on demand)
   void* scratch = nullptr;

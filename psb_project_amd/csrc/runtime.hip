@@ -349,8 +349,11 @@ psb_status psb_init(int32_t device, psb_context* out) {
     return PSB_ERR_NO_DEVICE;
   }
   PSB_HIP(hipSetDevice(device));
+  int cus = 0;
+  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   psb_context ctx = new psb_context_s();
   ctx->device = device;
+  ctx->cus = cus;
   hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
   if (e != hipSuccess) { delete ctx; return hip_fail(e, "hipStreamCreate", __FILE__, __LINE__); }
   e = hipMalloc(&ctx->d_flags, 64);

@@ -211,10 +211,8 @@ __global__ __launch_bounds__(256) void k_wcsph_forces_lanes(uint32_t n, Consts c
 template <bool STEP>
 static psb_status launch_wcsph_forces(uint32_t n, const Consts& c, bool surf, const uint32_t* cnt,
                                       const uint32_t* list, const float4* xs, const float4* vs,
-                                      const float* rho, const WcsphOut& o, hipStream_t s) {
-  int dev = 0, cus = 0;
-  PSB_HIP(hipGetDevice(&dev));
-  PSB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+                                      const float* rho, const WcsphOut& o, int cus,
+                                      hipStream_t s) {
   if (surf)
     hipLaunchKernelGGL((k_wcsph_forces<true, STEP>), dim3(blocks_for(n)), dim3(kBlock), 0, s, n, c,
                        cnt, list, xs, vs, rho, o);
@@ -316,12 +314,13 @@ psb_status launch_wcsph_step_forces(uint32_t n, const Consts& c, bool surf, cons
                                     const uint32_t* list, const float4* xs, const float4* vs,
                                     const float* rho, const float* pres, const float4* avh,
                                     const uint32_t* aid, float4* bx, float4* bv, float4* bvh,
-                                    uint32_t* bid, float* bp, uint32_t* flags, hipStream_t s) {
+                                    uint32_t* bid, float* bp, uint32_t* flags, int cus,
+                                    hipStream_t s) {
   if (!n) return PSB_OK;
   WcsphOut o{};
   o.bx = bx; o.bv = bv; o.bvh = bvh; o.bid = bid; o.bp = bp; o.avh = avh; o.aid = aid;
   o.pres = pres; o.flags = flags;
-  return launch_wcsph_forces<true>(n, c, surf, cnt, list, xs, vs, rho, o, s);
+  return launch_wcsph_forces<true>(n, c, surf, cnt, list, xs, vs, rho, o, cus, s);
 }
 
 }  // namespace psb
@@ -357,7 +356,7 @@ psb_status psb_evaluate_densities_forces(psb_context ctx, const psb_sph_params* 
   o.F = reinterpret_cast<float4*>(forces_accum4);
   PSB_HIP(hipGetLastError());
   return launch_wcsph_forces<false>(n, c, prm->surface_tension != 0.f, nb.count, nb.list, xs, vs,
-                                    density, o, ctx->stream);
+                                    density, o, ctx->cus, ctx->stream);
 }
 
 psb_status psb_force_constante(psb_context ctx, uint32_t n, float* accum4, const float* weight,

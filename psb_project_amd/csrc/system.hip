@@ -107,7 +107,6 @@ struct psb_system_s {
   float4* d_fb = nullptr;
   int sphere_cur = 0;
   int32_t corrector_lanes = 0;   // threads per particle in the corrector passes (0: by size)
-  int32_t cus = 0;               // compute units of the device
   std::vector<ColliderDev> colliders;   // after the box, in order
   ColliderDev* d_coll = nullptr;
   // per-particle materials (reference mode): table, material of each id,
@@ -285,7 +284,7 @@ static psb_status wcsph_step(psb_system s, int step) {
     Timed t(s, PH_FORCES, step);
     PSB_TRY(launch_wcsph_step_forces(s->n, s->c, s->prm.surface_tension != 0.f, s->ncount,
                                      s->nlist, s->ax, s->av, s->rho, s->pres, s->avh, s->aid, s->bx,
-                                     s->bv, s->bvh, s->bid, s->bp, s->flags, st));
+                                     s->bv, s->bvh, s->bid, s->bp, s->flags, s->ctx->cus, st));
   }
   return PSB_OK;
 }
@@ -365,7 +364,7 @@ static Lanes corrector_lanes(psb_system s) {
     return Lanes{l, l};
   }
   if (s->halo) return Lanes{1, 1};
-  const bool small = s->cus > 0 && (uint64_t)s->n <= 1024ull * (uint64_t)s->cus;
+  const bool small = (uint64_t)s->n <= 1024ull * (uint64_t)s->ctx->cus;
   const int l = small || s->grouped32 ? 2 : 1;
   return Lanes{l, l};
 }
@@ -483,7 +482,7 @@ static psb_status pcisph_attempt(psb_system s, int step, const Consts& c, bool f
   {
     Timed t(s, PH_NONPRESSURE, att);
     PSB_TRY(launch_pci_nonpressure(s->n, c, surf, warm, false, s->ncount, s->nlist, s->ax, s->av,
-                                   s->rho, s->avh, s->pres, b, o, st));
+                                   s->rho, s->avh, s->pres, b, o, s->ctx->cus, st));
   }
   float4* cur = s->xp0;
   float4* nxt = s->xp1;
@@ -634,10 +633,6 @@ psb_status psb_system_create(psb_context ctx, const psb_sph_params* prm, uint32_
   if (stt == PSB_OK) {
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) stt = hip_fail(e, "hipSetDevice", __FILE__, __LINE__);
-  }
-  if (stt == PSB_OK) {
-    hipError_t e = hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
-    if (e != hipSuccess) stt = hip_fail(e, "hipDeviceGetAttribute", __FILE__, __LINE__);
   }
   if (stt == PSB_OK) stt = grid_create(ctx, prm->grid, capacity, &s->grid);
   if (stt == PSB_OK) stt = sys_alloc(s);
