@@ -1,6 +1,7 @@
-"""The list walkers at the edges of their rounds: particles with 0 to 40
-neighbours in one wave (a random cloud), list capacities around a round's
-length, and particle counts around a wave's; bitwise against the oracle."""
+"""The list walkers at the edges of their rounds: particles with 1 to 40 list
+entries (themselves among them) in one wave (a random cloud), list capacities
+around a round's length, particle counts around a wave's, and waves with short
+lists beside some around and above 128 entries; bitwise against the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -67,4 +68,61 @@ def test_pcisph_steps_on_uneven_lists(ctx, oracle, n, mode, lanes):
             u, v = (a[k][:, :3], b[k][:, :3]) if a[k].ndim == 2 else (a[k], b[k])
             assert np.array_equal(u, v, equal_nan=True), k
     g.close()
+    o.close()
+
+
+def clusters(sizes, h, seed):
+    """Groups of particles within 0.35 h of one another, 3 h apart: lists of
+    exactly the groups' sizes, in the sorted order group after group."""
+    rng = np.random.default_rng(seed)
+    x = np.zeros((sum(sizes), 4), np.float32)
+    k = 0
+    for i, m in enumerate(sizes):
+        at = (np.array([i % 6, i // 6 % 6, i // 36]) * 3.0 + 1.0) * h
+        x[k:k + m, :3] = at + rng.uniform(0.0, 0.2 * h, (m, 3))
+        k += m
+    return x
+
+
+@pytest.mark.parametrize("mode", [MODE_REFERENCE, MODE_CONFIG])
+@pytest.mark.parametrize("sizes,cap", [
+    ((40, 127, 1, 2), 130), ((128, 3, 60), 130), ((5, 129, 1), 129), ((7, 131, 2), 130),
+    ((1, 127, 30, 128, 9, 129, 2, 130, 64, 1), 140), ((3, 260, 1, 390, 20), 400)])
+def test_long_lists_beside_short_ones(ctx, oracle, sizes, cap, mode):
+    p = scenes.pcisph_dam_break(n_side=1, mode=mode, retry_levels=0).params
+    p.max_neighbors, p.max_iterations, p.dt = cap, 4, 1e-7
+    x = clusters(sizes, p.support_radius, sum(sizes))
+    n = len(x)
+    r = gpu_grid_and_neighbors(ctx, x, p.grid, p.support_radius, cap)
+    assert sorted(r["count"].tolist()) == sorted(min(m, cap) for m in sizes for _ in range(m))
+    vel = np.zeros((n, 4), np.float32)
+    vel[:, :3] = np.random.default_rng(n).normal(scale=0.1, size=(n, 3))
+    dvel = ctx.to_device(vel)
+    outs = {k: ctx.array(16 * n) for k in ("normals", "fP", "fV", "fS", "F")}
+    rho, prs = ctx.array(4 * n), ctx.array(4 * n)
+    check(lib().psb_evaluate_densities_forces(
+        ctx.handle, C.byref(p), r["nb"], r["bufs"][1].ptr, dvel.ptr, n, rho.ptr, prs.ptr,
+        outs["normals"].ptr, outs["fP"].ptr, outs["fV"].ptr, outs["fS"].ptr, outs["F"].ptr))
+    ref = oracle.evaluate_densities_forces(p, r["count"], r["list"].ravel(), r["xs"], vel)
+    assert np.array_equal(rho.download(np.float32, n), ref["density"])
+    assert np.array_equal(prs.download(np.float32, n), ref["pressure"])
+    for k in outs:
+        assert np.array_equal(outs[k].download(np.float32, (n, 4))[:, :3], ref[k][:, :3],
+                              equal_nan=True), k
+    # pci_SPH_update over the same lists, against one step of the oracle
+    z = np.zeros((n, 4), np.float32)
+    d = {k: ctx.to_device(v) for k, v in dict(old=z, pos=r["xs"], vel=z, vav=z, vap=z).items()}
+    prs.zero()
+    its, err = C.c_int32(), C.c_float()
+    check(lib().psb_pci_sph_update(ctx.handle, C.byref(p), r["nb"], d["old"].ptr, d["pos"].ptr,
+                                   d["vel"].ptr, d["vav"].ptr, d["vap"].ptr, rho.ptr, prs.ptr,
+                                   None, None, None, None, None, n, C.byref(its), C.byref(err)))
+    o = oracle.OracleSystem(p, n)
+    o.set_particles(x)
+    o.update(1)
+    ref, st = o.state(), o.stats()
+    assert its.value == st["iterations"]
+    assert np.float32(err.value) == np.float32(st["max_error"])
+    assert np.array_equal(rho.download(np.float32, n), ref["density"])
+    assert np.array_equal(prs.download(np.float32, n), ref["pressure"])
     o.close()
