@@ -989,25 +989,28 @@ psb_status launch_neighbors(psb_grid g, const float4* xs, uint32_t n, float r2, 
   if (ep && rho) e = *ep;
   // Several lanes per particle, for the stencils that have that kernel, while
   // one leaves the chip short of waves.  Us, one lane -> kSplit, cells of half
-  // the radius (cells of the radius):
-  //   with the density sum     cube           4 layers       2 layers
-  //      4,096              27 -> 9 (34, 10)
-  //     47,000              28 -> 15 (35, 16)  25 -> 16 (27, 15)  17 -> 14 (17, 14)
-  //     64,000              29 -> 19 (37, 24)  26 -> 20 (28, 21)  19 -> 19 (19, 20)
-  //     97,000              33 -> 29 (41, 31)  27 -> 28 (32, 30)  21 -> 26 (21, 27)
-  //    125,000              33 -> 34 (42, 39)  28 -> 34 (33, 38)  22 -> 30 (23, 34)
+  // the radius (cells of the radius); blocks and sheets as loaded (a lattice),
+  // and after some hundred steps, when the lanes of a wave have rows of
+  // different lengths:
+  //   with the density sum     block           4 layers        2 layers
+  //      4,096 loaded        27 -> 9 (34, 10)
+  //     64,000 loaded        29 -> 19 (37, 24)  26 -> 20 (28, 21)  19 -> 19 (19, 20)
+  //     64,000 moved         50 -> 27 (60, 28)  45 -> 24 (53, 25)  29 -> 18 (28, 18)
+  //    125,000 loaded        33 -> 34 (42, 39)  28 -> 34 (33, 38)  22 -> 30 (23, 34)
+  //    125,000 moved         56 -> 45 (67, 45)  50 -> 39 (58, 41)  30 -> 28 (31, 29)
+  //    146,000 moved         64 -> 51 (77, 50)  52 -> 40 (66, 45)  32 -> 31 (32, 31)
   //   without
-  //    148,000              35 -> 22 (46, 30)  29 -> 21 (36, 23)  24 -> 19 (25, 19)
-  //    262,144              41 -> 34 (57, 42)  36 -> 32 (46, 37)  29 -> 29 (32, 30)
-  //    512,000              72 -> 68 (99, 85)  63 -> 65 (76, 76)  48 -> 59 (47, 65)
-  // With the sum the line lies at 97,000, and at 65,536 where the lists are long
+  //    148,000 loaded        35 -> 22 (46, 30)  29 -> 21 (36, 23)  24 -> 19 (25, 19)
+  //    262,144 loaded        41 -> 34 (57, 42)  36 -> 32 (46, 37)  29 -> 29 (32, 30)
+  //    512,000 loaded        72 -> 68 (99, 85)  63 -> 65 (76, 76)  48 -> 59 (47, 65)
+  // With the sum the line lies at 147,456, and at 65,536 where the lists are long
   // enough for neighbour counts that do not fit the lanes' buffers: 145
   // neighbours 123 -> 67 at 47,000, 148 -> 151 at 97,000; 268 (cells of half the
   // radius; of the radius) 142 -> 63 (234, 92) at 8,000, 241 -> 231 (331, 273) at
   // 47,000, 259 -> 323 (356, 412) at 64,000.  Without it at 262,144 (268: 477 ->
   // 452).  Staged tiles keep the plain search, and so do particles whose index
   // takes more than 24 bits.
-  const uint64_t per_cu = !rho ? 1024u : nb.capacity <= 192u ? 384u : 256u;
+  const uint64_t per_cu = !rho ? 1024u : nb.capacity <= 192u ? 576u : 256u;
   if (!tiles && (R == 1 || R == 2) && n < 1u << 24 && n <= per_cu * (uint64_t)g->ctx->cus) {
 #define PSB_NBS(D_, R_)                                                                           \
   hipLaunchKernelGGL((k_neighbors_split<D_, R_>), dim3(blocks_for(n, 64u)),                       \

@@ -167,14 +167,14 @@ def test_long_lists(ctx, oracle, h, width):
 
 
 @pytest.mark.parametrize("width", [1, 2])
-@pytest.mark.parametrize("n,cap,solver", [(98304, 96, "wcsph"), (98305, 96, "wcsph"),
-                                          (98305, 17, "pcisph"), (65536, 200, "pcisph"),
+@pytest.mark.parametrize("n,cap,solver", [(147456, 96, "wcsph"), (147457, 96, "wcsph"),
+                                          (147457, 17, "pcisph"), (65536, 200, "pcisph"),
                                           (65537, 200, "pcisph")])
 def test_both_sides_of_the_rule(ctx, oracle, n, cap, solver, width):
-    """Counts where a lane per particle takes over (384 and, for longer lists,
+    """Counts where a lane per particle takes over (576 and, for longer lists,
     256 particles a compute unit), with whole and with cut-off lists."""
-    p = lattice_params((47, 47, 45), width, solver, cap)
-    steps_equal(ctx, oracle, p, lattice((47, 47, 45), n)[:n], steps=1)
+    p = lattice_params((54, 53, 52), width, solver, cap)
+    steps_equal(ctx, oracle, p, lattice((54, 53, 52), n)[:n], steps=1)
 
 
 @pytest.mark.parametrize("width", [1, 2])
