@@ -103,18 +103,19 @@ struct NodeGrid {
   int nx, ny, nz;
   float ox, oy, oz, cell;
   float iso, r2, inv_r6;
-  float edge2;   // near_edge of r2
 };
 
-// The d^2 above which a particle closer than r may lie outside a point's 27
-// cells.  An index (x - min) / r carries two roundings, so it is off by at most
-// 2^-23 of itself: of two points in a grid of `cells` along its longest axis
-// the one more than a cell away is no nearer than (1 - 2^-22 cells) r.  Above
-// 2,000 cells that is less than 0.999 of r^2, which 16,000 cells do pass.
-inline float near_edge(float r2, int cells) {
-  const double share = 1.0 - (double)cells / (1 << 21) - 1.0 / (1 << 18);
-  return r2 * (float)std::max(0.0, std::min(0.999, share));
-}
+constexpr int kMaxNodes = 4096;   // per axis
+// A wave takes its block's candidates together up to this node spacing over
+// r; above, each lane walks its own 27 cells.  The box a wave has to look
+// through grows with the cube of (3 spacings + 2 r), a lane's cells do not.
+// Us per extraction, box / cells (particles; r in particle spacings):
+//                    0.25         0.4        0.5        1          4
+//   262,144; 3.1   336 / 443   275 / 298  308 / 246  850 / 253  10,450 / 219
+//   32,768; 3.1    200 / 208   264 / 218  275 / 208  777 / 230   5,860 / 214
+//   262,144; 2     340 / 423   220 / 274  208 / 195  321 / 156   2,400 / 141
+//   32,768; 5                  607 / 522  780 / 500  2,265 / 520
+constexpr float kBoxCells = 0.4f;
 
 __device__ __forceinline__ void node_pos(const NodeGrid& G, int i, int j, int k, float& x, float& y,
                                          float& z) {
@@ -160,10 +161,10 @@ __device__ __forceinline__ void box_cells(const GridDev& g, WaveBox& w) {
 // of the box go to LDS in order, and every lane then sees each of them (an
 // LDS broadcast).  The field and normal sums of a lane's own 27 cells are
 // ~780 candidates at r = 3 spacings of which ~120 lie within r; per wave ~620
-// are near a block of 4^3 nodes a third of r apart, and one load serves 64 nodes instead of a
-// gather (through the permutation) per candidate and node.  262,144 particles,
-// 440,000 nodes: k_iso 617 -> 106 us, k_vertices 245 -> 57 us; what is left
-// is the ~13 VALU instructions per wave and survivor.
+// are near a block of 4^3 nodes a third of r apart, and one load serves 64 nodes
+// instead of a gather (through the permutation) per candidate and node.  262,144
+// particles, 440,000 nodes: k_iso 617 -> 106 us, k_vertices 245 -> 57 us; what
+// is left is the ~13 VALU instructions per wave and survivor.
 template <class F>
 __device__ __forceinline__ void for_near_box(const GridDev& g, const uint32_t* __restrict__ start,
                                              const float4* __restrict__ xs, const WaveBox& w,
@@ -204,7 +205,13 @@ __device__ __forceinline__ void for_near_box(const GridDev& g, const uint32_t* _
 
 // Whether particle x lies in the 27 cells around the point whose cell is c.  A
 // particle outside them is more than a cell (r) away but for rounding at the
-// cell borders: only a d^2 above NodeGrid::edge2 needs the test (near_edge).
+// cell borders: only a distance this close to r needs the test.  An index
+// (x - min) / r carries two roundings, so it is off by at most 2^-23 of itself:
+// of two points in a grid of N cells along an axis the one more than a cell away
+// is no nearer than (1 - 2^-22 N) r.  Where nodes are close enough for the block
+// kernels N is at most 1,640; from 16,000 on the rounding does pass 0.999 of r^2.
+constexpr float kNearEdge = 0.999f;
+static_assert((kBoxCells * kMaxNodes + 2) / (1 << 21) + 1.f / (1 << 18) < 1.f - kNearEdge, "kNearEdge");
 __device__ __forceinline__ bool in_cells(const GridDev& g, const int (&c)[3], const float4& x) {
   uint32_t bad = 0;
   const int kx = cell_coord(x.x, g.minx, g.cell, g.nx, bad);
@@ -220,8 +227,7 @@ __device__ __forceinline__ void cells_of(const GridDev& g, float x, float y, flo
 }
 
 // The same for each lane by itself: the particles of the 27 cells around c in
-// sorted order, four loads in flight (at one spacing per cell bound by their
-// latency).
+// sorted order, four loads in flight.
 template <class F>
 __device__ __forceinline__ void for_near_cells(const GridDev& g, const uint32_t* __restrict__ start,
                                                const float4* __restrict__ xs, const int (&c)[3],
@@ -292,7 +298,7 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_iso(NodeGrid G, GridDev g,
   node_pos(G, o[0], o[1], o[2], w.lo[0], w.lo[1], w.lo[2]);
   node_pos(G, e[0], e[1], e[2], w.hi[0], w.hi[1], w.hi[2]);
   box_cells(g, w);
-  const float edge2 = G.edge2;
+  const float edge2 = G.r2 * kNearEdge;
   for_near_box(g, start, xs, w, G.r2, lds[wv], [&](const float4& q) {
     const float dx = x - q.x, dy = y - q.y, dz = z - q.z;
     const float d2 = dot3(dx, dy, dz, dx, dy, dz);
@@ -304,17 +310,6 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_iso(NodeGrid G, GridDev g,
   if (mine)
     iso[(uint64_t)i + (uint64_t)G.nx * ((uint64_t)j + (uint64_t)G.ny * (uint64_t)k)] = acc * G.inv_r6;
 }
-
-// A wave takes its block's candidates together up to this node spacing over
-// r; above, each lane walks its own 27 cells.  The box a wave has to look
-// through grows with the cube of (3 spacings + 2 r), a lane's cells do not.
-// Us per extraction, box / cells (particles; r in particle spacings):
-//                    0.25         0.4        0.5        1          4
-//   262,144; 3.1   336 / 443   275 / 298  308 / 246  850 / 253  10,450 / 219
-//   32,768; 3.1    200 / 208   264 / 218  275 / 208  777 / 230   5,860 / 214
-//   262,144; 2     340 / 423   220 / 274  208 / 195  321 / 156   2,400 / 141
-//   32,768; 5                  607 / 522  780 / 500  2,265 / 520
-constexpr float kBoxCells = 0.4f;
 
 __global__ __launch_bounds__(256) void k_edges(NodeGrid G, const float* __restrict__ iso,
                                                uint8_t* __restrict__ eflags,
@@ -367,7 +362,7 @@ __global__ __launch_bounds__(64 * kIsoWaves) void k_vertices(
     node_pos(G, o[0] + kNodeBlock, o[1] + kNodeBlock, o[2] + kNodeBlock, w.hi[0], w.hi[1], w.hi[2]);
     box_cells(g, w);
   }
-  const float edge2 = G.edge2;
+  const float edge2 = G.r2 * kNearEdge;
   for (uint32_t v0 = 0; v0 < total; v0 += 64u) {
     const bool on = v0 + lane < total;
     const uint32_t ed = edge[wv][on ? v0 + lane : v0];
@@ -624,7 +619,7 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
     mx[a] = (double)hi[a] + margin;
     const double len = std::fabs(mx[a] - mn[a]);
     const double nd = std::ceil(len / (double)prm->cell_size);
-    PSB_ARG(nd >= 2 && nd <= 4096, "surface node grid must have 2..4096 nodes per axis");
+    PSB_ARG(nd >= 2 && nd <= kMaxNodes, "surface node grid must have 2..4096 nodes per axis");
     dims[a] = (uint32_t)nd;
     const double center = (mn[a] + mx[a]) / 2;
     org[a] = (float)(center - len / 2 + (double)prm->cell_size / 2);
@@ -647,7 +642,6 @@ psb_status psb_surface_extract_points(psb_surface s, const float* pos4, const ui
   gd.cell_size = r;
   PSB_ARG((uint64_t)gd.dims[0] * gd.dims[1] * gd.dims[2] <= (1ull << 31),
           "particle grid too fine for the surface radius");
-  G.edge2 = near_edge(G.r2, std::max(gd.dims[0], std::max(gd.dims[1], gd.dims[2])));
   if (!s->grid || std::memcmp(&gd, &s->gdesc, sizeof gd) != 0 || n > s->grid_cap) {
     if (s->grid) { psb_finalize_grid(s->grid); s->grid = nullptr; }
     PSB_TRY(psb_create_grid_desc(s->ctx, &gd, n, &s->grid));
